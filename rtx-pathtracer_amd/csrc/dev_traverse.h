@@ -294,10 +294,10 @@ RTX_DI bool alphaAccept(const LaneScene &S, int prim, float ox, float t, float b
 // ------------------------------------------------------------------
 // Persistent traversal with lane refill (Aila & Laine 2009, sections 4-5):
 // each wave loops until the queue is drained; lanes whose ray finished
-// fetch a new ray (one atomic per wave), and the "while-while" loop with
-// postponed leaves keeps lanes in step: a lane that reaches a leaf parks
-// it and keeps descending until every lane of the wave has a leaf, then
-// the wave intersects leaves together.
+// fetch a new ray, and node visits and leaf tests alternate with postponed
+// leaves: a lane that reaches a leaf parks it and keeps descending until
+// enough of the wave's lanes wait at a leaf, then those are intersected
+// together.
 struct LaneRay {
     TravRay r;
     float tmin, tmax, bu, bv;
@@ -381,13 +381,40 @@ template <int HIT, class SceneT> RTX_DI void beginRay(const SceneT &S, LaneRay &
 // L.any under kHitLane); S is the scene (a DevScene for launches over one
 // scene, or a per-lane LaneScene that load() points at the ray's scene);
 // store(L) consumes a finished ray.  `fetch` must be zero at launch.  Each
-// wave first takes its own 64 rays of the grid's static span (thread i of
-// the grid: ray i) without an atomic, so a launch over a short or empty queue
-// costs no contention; after that a wave refills when at least kRefillLanes
-// of its lanes are idle (or all are), with one atomic for the whole wave on
-// the rays past the static span.  Once the queue is drained the wave stops
-// fetching, so `fetch` ends below n + 64 * waves.
-constexpr int kRefillLanes = 16;
+// wave first takes its own slice of up to 64 rays of the grid's static span
+// without an atomic, so a launch over a short or empty queue costs no
+// contention; the rays past the static span go out in chunks, one atomic a
+// chunk, and the wave refills its idle lanes from the chunk it holds whenever
+// at least kRefillLanes of them are idle (or all are).
+//
+// A short queue is bound by the latency of its longest rays, and every node
+// or leaf step of a lane's neighbours lengthens its own chain: so a queue that
+// would not fill the waves is spread over 1 / kSpread of them, a few rays
+// each.  Closest hits through the host call, 2047 rays in the 262,144-triangle
+// room: 134 us with 64 rays a wave, 105 us spread (8191: 158 and 129); 1080p
+// cache frames, whose last bounces are short, 452 and 442 ms for 44 frames.
+// Over all the waves, 30,000 and more rays in a small scene lost up to 30%
+// (three times the wave steps); over a quarter or an eighth of them the large
+// scene's 8191 rays lost 7 to 11%.
+//
+// The work counter is one word that every XCD updates, so its atomics are
+// served one after another, a few nanoseconds each: with one a refill (about
+// 20 rays) they bounded a 4.1 M-ray launch at 1.85 ms.  A chunk is a
+// kChunksPerWave-th of a wave's share of the rest, so that the waves end
+// together, at least a whole wave's worth and at most kChunkMax: 8 chunks of
+// at most 512 rays took that launch to 1.49 ms (32 of at most 256, or 4 of at
+// most 1024, within 0.5% of it).
+// Once the queue is drained the wave stops fetching, so `fetch` ends below
+// n + kChunkMax * waves.
+constexpr int kRefillLanes = 24;          // 16 to 32: within 0.3% of each other; 8: 1% slower
+constexpr uint32_t kChunksPerWave = 8, kChunkMax = 512;
+constexpr uint32_t kSpread = 2;
+// Inner nodes are visited while at least kNodeNum / kNodeDen of the active
+// lanes have one to visit; then every lane that holds a leaf intersects it.
+// A ray visits some ten inner nodes a leaf, so waiting until every lane holds
+// a leaf left two thirds of the lanes idle.  1/2 measured the same, 7/8 1-2%
+// slower (more leaf passes over few lanes).
+constexpr int kNodeNum = 3, kNodeDen = 4;
 
 template <int HIT, bool COUNT, bool ALPHA, class SceneT, class Stack, class Load, class Store>
 RTX_DI void persistentTrace(const SceneT &S, uint32_t n, uint32_t *fetch, Stack &st, VisitCount &vc, Load load,
@@ -397,10 +424,15 @@ RTX_DI void persistentTrace(const SceneT &S, uint32_t n, uint32_t *fetch, Stack 
     L.idx = 0;
     L.any = HIT == kHitAny;
     bool active = false;
-    bool drained = false; // wave-uniform
-    bool first = true;    // wave-uniform
-    const uint32_t staticSpan = gridDim.x * blockDim.x; // blockDim.x is a multiple of 64
-    const uint32_t waveBase = blockIdx.x * blockDim.x + (threadIdx.x & ~63u);
+    bool first = true, last = false, drained = false; // wave-uniform: no chunk yet, none after this one, none left
+    const uint32_t waves = gridDim.x * (blockDim.x >> 6); // blockDim.x is a multiple of 64
+    const uint32_t spread = max(waves / kSpread, 1u);
+    const uint32_t slice = min(n / spread + (n % spread != 0u ? 1u : 0u), 64u);
+    const uint32_t staticSpan = waves * slice;
+    const uint32_t waveBase = (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * slice;
+    uint32_t cur = 0, end = 0; // wave-uniform: the chunk of rays the wave still holds
+    const uint32_t chunk =
+        n <= staticSpan ? 64u : min(max((n - staticSpan) / (waves * kChunksPerWave), 64u), kChunkMax);
     for (;;) {
         // refill idle lanes (the whole wave is converged here)
         const bool idle = !active;
@@ -409,21 +441,30 @@ RTX_DI void persistentTrace(const SceneT &S, uint32_t n, uint32_t *fetch, Stack 
         const bool anyActive = nIdle < 64; // gfx950 waves are 64 wide; blocks are whole waves
         if (!drained && (nIdle >= kRefillLanes || !anyActive)) {
             const int lane = (int)__lane_id();
-            uint32_t base = 0;
-            if (first) { // every lane idle: the wave's static slice
-                first = false;
-                base = waveBase;
-                if (staticSpan >= n) drained = true;
-            } else {
-                const int leader = __ffsll((unsigned long long)m) - 1;
-                if (lane == leader) base = atomicAdd(fetch, (uint32_t)nIdle);
-                base = staticSpan + __shfl(base, leader);
-                if (base + (uint32_t)nIdle >= n) drained = true;
+            if (cur == end) { // the wave's chunk is used up
+                if (first) { // every lane idle: the wave's static slice
+                    first = false;
+                    cur = waveBase;
+                    end = waveBase + slice;
+                    last = staticSpan >= n;
+                } else {
+                    uint32_t base = 0;
+                    if (lane == 0) base = atomicAdd(fetch, chunk);
+                    cur = staticSpan + __builtin_amdgcn_readfirstlane(base);
+                    end = cur + chunk;
+                    last = end >= n;
+                }
+                end = min(end, n);
+                cur = min(cur, end);
             }
+            const uint32_t base = cur;
+            const uint32_t take = min((uint32_t)nIdle, end - cur);
+            cur += take;
+            drained = last && cur == end;
             if (idle) {
                 const uint64_t below = lane == 0 ? 0ull : (m & ((~0ull) >> (64 - lane)));
-                const uint32_t idx = base + (uint32_t)__popcll(below);
-                if (idx < n) {
+                const uint32_t rank = (uint32_t)__popcll(below), idx = base + rank;
+                if (rank < take) {
                     L.idx = idx;
                     load(idx, L);
                     st.sp = 0;
@@ -432,34 +473,36 @@ RTX_DI void persistentTrace(const SceneT &S, uint32_t n, uint32_t *fetch, Stack 
                 }
             }
         }
-        if (__ballot(active) == 0) break;
-        if (active) {
-            // inner nodes until every lane of the wave holds a leaf (or is done)
-            while (L.link >= 0) {
+        const int nActive = __popcll(__ballot(active));
+        if (nActive == 0) break;
+        // inner nodes while most of the active lanes have one to visit
+        int nNode;
+        do {
+            if (L.link >= 0) {
                 L.link = innerStep<COUNT>(S, L, st, vc);
                 if (L.link < 0 && L.link != kLinkDone && L.leaf == kLinkDone) {
                     L.leaf = L.link;
                     L.link = popOrDone(st);
                 }
-                if (__ballot(L.leaf == kLinkDone) == 0) break;
             }
-            // leaves
-            while (L.leaf != kLinkDone) {
-                if (leafStep<HIT, COUNT, ALPHA>(S, L, L.leaf, vc)) {
-                    L.link = kLinkDone;
-                    L.leaf = kLinkDone;
-                    break;
-                }
+            nNode = __popcll(__ballot(L.link >= 0));
+        } while (nNode * kNodeDen >= nActive * kNodeNum && nNode > 0);
+        // one leaf of every lane that holds one
+        if (L.leaf != kLinkDone) {
+            if (leafStep<HIT, COUNT, ALPHA>(S, L, L.leaf, vc)) {
+                L.link = kLinkDone;
+                L.leaf = kLinkDone;
+            } else {
                 L.leaf = kLinkDone;
                 if (L.link < 0 && L.link != kLinkDone) {
                     L.leaf = L.link;
                     L.link = popOrDone(st);
                 }
             }
-            if (L.link == kLinkDone && L.leaf == kLinkDone) {
-                store(L);
-                active = false;
-            }
+        }
+        if (active && L.link == kLinkDone && L.leaf == kLinkDone) {
+            store(L);
+            active = false;
         }
     }
 }
