@@ -413,8 +413,8 @@ typedef struct rtx_tuning {
                                  7 waves per SIMD) */
     int32_t shadeBlocksPerCU; /* 256-thread shading blocks per CU (default 8) */
     uint32_t batchPaths;      /* paths in flight per batch when rtx_frame_params.batchPaths is 0 (2^22) */
-    int32_t ldsStackEntries;  /* traversal stack entries per thread held in LDS: 12, 16, 20 or 24
-                                 (20); deeper entries spill to scratch */
+    int32_t ldsStackEntries;  /* 4-byte words of the traversal stack per thread held in LDS: 12, 16,
+                                 20 or 24 (20; an entry takes two); deeper entries spill to scratch */
     int32_t cacheUpkeep;      /* irradiance-cache frames: 1 = the update jobs' sub-paths run in
                                  the frame's own bounces, beside its camera paths, where the
                                  path buffers hold both (default); 2 = every job after the

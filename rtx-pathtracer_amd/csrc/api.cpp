@@ -552,9 +552,14 @@ int rtx_scene_create(rtx_ctx *ctx, const rtx_scene_desc *d, rtx_scene **out) try
             primRef[t] = make_int2((int)i, (int)f);
         }
     }
-    BvhBuildResult bvh;
+    WideBvh bvh;
+    double buildMs = 0.0;
     try {
-        buildBvh(tv.data(), (uint32_t)numTris, bvh);
+        BvhBuildResult tree;
+        buildBvh(tv.data(), (uint32_t)numTris, tree);
+        const auto t0 = std::chrono::steady_clock::now();
+        packWide(tree, bvh);
+        buildMs = tree.buildMs + std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     } catch (const std::exception &e) {
         return fail(ctx, RTX_E_INVALID, std::string("BVH build failed: ") + e.what());
     }
@@ -572,8 +577,8 @@ int rtx_scene_create(rtx_ctx *ctx, const rtx_scene_desc *d, rtx_scene **out) try
         }
     }
     std::vector<float4> tris((size_t)numTris * 3);
-    for (size_t k = 0; k < bvh.primOrder.size(); ++k) {
-        uint32_t p = bvh.primOrder[k];
+    for (size_t k = 0; k < bvh.triOrder.size(); ++k) {
+        uint32_t p = bvh.triOrder[k];
         const float *v = &tv[9 * (size_t)p];
         int pid = (int)p | (alpha[p] ? kAlphaBit : 0);
         float pidBits;
@@ -586,8 +591,8 @@ int rtx_scene_create(rtx_ctx *ctx, const rtx_scene_desc *d, rtx_scene **out) try
     // their light first: kept only while few and none is alpha-tested
     std::vector<float4> lightTris;
     bool lightTrisOk = true;
-    for (size_t k = 0; k < bvh.primOrder.size() && lightTrisOk; ++k) {
-        const uint32_t p = bvh.primOrder[k];
+    for (size_t k = 0; k < bvh.triOrder.size() && lightTrisOk; ++k) {
+        const uint32_t p = bvh.triOrder[k];
         const rtx_instance &in = d->instances[primRef[p].x];
         const rtx_model_desc &md = d->models[in.modelIndex];
         const int mat = md.vertices[md.indices[3 * (size_t)primRef[p].y]].materialIndex;
@@ -629,7 +634,7 @@ int rtx_scene_create(rtx_ctx *ctx, const rtx_scene_desc *d, rtx_scene **out) try
     int32_t *liD = nullptr;
     rtx_face_sample *ftD = nullptr;
     rtx_sphere *spD = nullptr;
-    if (e == hipSuccess) e = upload(&nodes, reinterpret_cast<const float4 *>(bvh.nodes.data()), bvh.nodes.size() * 8);
+    if (e == hipSuccess) e = upload(&nodes, reinterpret_cast<const float4 *>(bvh.nodes.data()), bvh.nodes.size() * kWideNodeSlots);
     if (e == hipSuccess) e = upload(&trisD, tris.data(), tris.size());
     float4 *lightTrisD = nullptr;
     if (e == hipSuccess && lightTrisOk && !lightTris.empty()) e = upload(&lightTrisD, lightTris.data(), lightTris.size());
@@ -747,10 +752,10 @@ int rtx_scene_create(rtx_ctx *ctx, const rtx_scene_desc *d, rtx_scene **out) try
     sc->info.spheres = d->sphereCount;
     sc->info.nodes = (uint32_t)bvh.nodes.size();
     sc->info.maxDepth = bvh.maxDepth;
-    sc->info.deviceBytes = bvh.nodes.size() * sizeof(Bvh4Node) + tris.size() * sizeof(float4) +
+    sc->info.deviceBytes = bvh.nodes.size() * sizeof(Bvh8Node) + tris.size() * sizeof(float4) +
                            primRef.size() * sizeof(int4) + verts.size() * sizeof(rtx_vertex) +
                            idx.size() * 4 + (size_t)d->materialCount * sizeof(rtx_material);
-    sc->info.buildMs = bvh.buildMs;
+    sc->info.buildMs = buildMs;
     for (int a = 0; a < 3; ++a) {
         sc->info.boundsMin[a] = std::numeric_limits<float>::infinity();
         sc->info.boundsMax[a] = -std::numeric_limits<float>::infinity();
@@ -1388,7 +1393,7 @@ int rtx_render(rtx_ctx *ctx, const rtx_scene *scene, const rtx_frame_params *p, 
         }
         stats->batches = batches;
         stats->bounces = (uint32_t)itersRun;
-        stats->nodeBytes = kBvh4NodeBytesRead;
+        stats->nodeBytes = kWideNodeBytes;
         stats->primBytes = 48;
     }
     return RTX_OK;

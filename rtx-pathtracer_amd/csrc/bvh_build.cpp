@@ -1,7 +1,7 @@
 // Host BVH builder: binned surface-area heuristic (Wald, "On fast
 // construction of SAH-based bounding volume hierarchies", 2007) for a
-// binary tree, collapsed into the four-wide nodes the traversal kernels read.  It replaces the
-// driver's BLAS/TLAS build (src/SceneLoader.cpp:1101-1193), whose source
+// binary tree, collapsed into four-wide nodes (bvh_wide.cpp packs those into
+// the nodes the traversal kernels read).  It replaces the driver's BLAS/TLAS build (src/SceneLoader.cpp:1101-1193), whose source
 // is not available.
 #include <algorithm>
 #include <chrono>
@@ -50,6 +50,7 @@ struct Box {
 constexpr int kBins = 64;
 constexpr int kSahDepthLimit = 32; // deeper subtrees use object-median splits
 constexpr int kLeafTarget = 1;
+constexpr uint32_t kSmallCount = 24; // subtrees searched primitive by primitive
 
 struct Builder {
     std::vector<Box> primBox;
@@ -57,6 +58,47 @@ struct Builder {
     std::vector<uint32_t> order;
     std::vector<BvhNode> nodes;
     uint32_t maxDepth = 0;
+
+    // The binned search on axis a for a few primitives: sorted by bin, only
+    // the bins that hold one are visited.  An empty bin's cut costs what the
+    // cut before it does and is never taken, so the choice is the full
+    // search's; resetting and sweeping 64 bins for the many small subtrees
+    // was most of the build.
+    void sweepSmall(uint32_t start, uint32_t count, int a, float lo, float scale, float &bestCost, int &bestAxis,
+                    int &bestBin) const {
+        int bin[kSmallCount];
+        uint32_t prim[kSmallCount];
+        for (uint32_t i = 0; i < count; ++i) {
+            const uint32_t p = order[start + i];
+            int b = (int)((centroid[3 * (size_t)p + a] - lo) * scale);
+            b = std::min(std::max(b, 0), kBins - 1);
+            uint32_t k = i;
+            for (; k > 0 && bin[k - 1] > b; --k) {
+                bin[k] = bin[k - 1];
+                prim[k] = prim[k - 1];
+            }
+            bin[k] = b;
+            prim[k] = p;
+        }
+        float right[kSmallCount]; // area of primitives k.. on
+        Box acc;
+        acc.reset();
+        for (uint32_t k = count; k-- > 1;) {
+            acc.grow(primBox[prim[k]]);
+            right[k] = acc.area();
+        }
+        acc.reset();
+        for (uint32_t k = 0; k + 1 < count; ++k) {
+            acc.grow(primBox[prim[k]]);
+            if (bin[k] == bin[k + 1]) continue;
+            const float cost = acc.area() * (k + 1) + right[k + 1] * (count - k - 1);
+            if (cost < bestCost) {
+                bestCost = cost;
+                bestAxis = a;
+                bestBin = bin[k];
+            }
+        }
+    }
 
     // Returns the link for the subtree over order[start, start+count).
     int32_t build(uint32_t start, uint32_t count, uint32_t depth, Box &outBox) {
@@ -85,6 +127,10 @@ struct Builder {
             for (int a = 0; a < 3; ++a) {
                 float ext = cbox.hi[a] - cbox.lo[a];
                 if (!(ext > 0.0f)) continue;
+                if (count <= kSmallCount) {
+                    sweepSmall(start, count, a, cbox.lo[a], kBins / ext, bestCost, bestAxis, bestBin);
+                    continue;
+                }
                 Box bb[kBins];
                 uint32_t bc[kBins] = {0};
                 for (auto &b : bb) b.reset();
@@ -283,6 +329,7 @@ void buildBvh(const float *tv, uint32_t numTris, BvhBuildResult &out) {
         Builder::setNode(b.nodes.back(), all, empty, root, makeLeaf(0, 1));
         b.maxDepth = 0;
     }
+    out.scale = S;
     out.binaryDepth = b.maxDepth + 1;
     Collapser c{b.nodes, {}, 0};
     c.collapse(0, 1);

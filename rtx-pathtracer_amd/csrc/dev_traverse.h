@@ -3,11 +3,11 @@
 // shadow any-hit with TerminateOnFirstHit: raytrace.rgen:622-638) and the
 // sphere intersection shader (raytrace.sphere.rint:11-29).
 //
-// Stack-based traversal (Aila & Laine 2009) over four-wide nodes; the
-// stack's first LDS_DEPTH entries live in LDS (one column per thread, so
-// consecutive lanes hit consecutive banks), deeper entries in a private
-// array.  The builder bounds the stack use (3 entries per level) by
-// kStackCapacity.
+// Stack-based traversal (Aila & Laine 2009) over eight-wide quantised nodes
+// (csrc/bvh.h).  The stack's first LDS_DEPTH entries live in LDS (one column
+// per thread, so consecutive lanes hit consecutive banks), deeper entries in
+// a private array; an entry is one node's children still to visit, so the
+// stack holds at most one a level (kStackCapacity).
 #pragma once
 
 #include "dev_math.h"
@@ -18,7 +18,10 @@ namespace rtx {
 
 struct TravRay {
     V3 o, d, inv;
-    V3 oinv; // o * inv: slab plane distances are fma(l, inv, -oinv)
+    V3 oinv; // o * inv: a plane at l is fma(l, inv, -oinv) away
+    // the slots a node's children are looked at in first, by the ray's signs:
+    // of each half, quarter and pair (WideBvh's slot order)
+    uint32_t near4, near2, near1;
     int kx, ky, kz;
     float Sx, Sy, Sz;
 };
@@ -33,6 +36,9 @@ RTX_DI TravRay makeTravRay(V3 o, V3 d) {
     float dz = d.z != 0.0f ? d.z : copysignf(1e-30f, d.z);
     r.inv = v3(1.0f / dx, 1.0f / dy, 1.0f / dz);
     r.oinv = v3(o.x * r.inv.x, o.y * r.inv.y, o.z * r.inv.z);
+    r.near1 = r.inv.x < 0.0f ? 0xAAu : 0x55u;
+    r.near2 = r.inv.y < 0.0f ? 0xCCu : 0x33u;
+    r.near4 = r.inv.z < 0.0f ? 0xF0u : 0x0Fu;
     // watertight test set-up (Woop, Benthin, Wald, JCGT 2013)
     float ax = fabsf(d.x), ay = fabsf(d.y), az = fabsf(d.z);
     int kz = (ax > ay) ? (ax > az ? 0 : 2) : (ay > az ? 1 : 2);
@@ -51,21 +57,6 @@ RTX_DI TravRay makeTravRay(V3 o, V3 d) {
     r.Sy = sel(d, ky) / dkz;
     r.Sz = 1.0f / dkz;
     return r;
-}
-
-// Slab test against [lo, hi]: plane distances as one FMA each,
-// fma(l, inv, -o * inv); the absolute part of its error (o * inv rounded) is
-// covered by the builder's box padding (bvh_build.cpp), the relative part by
-// the 1 + 2*gamma_3 factor of Ize, "Robust BVH ray traversal" (JCGT 2013).
-RTX_DI bool slab(float lx, float ly, float lz, float hx, float hy, float hz, const TravRay &r, float tmin,
-                 float tmax, float &tnear) {
-    float tx0 = fmaf(lx, r.inv.x, -r.oinv.x), tx1 = fmaf(hx, r.inv.x, -r.oinv.x);
-    float ty0 = fmaf(ly, r.inv.y, -r.oinv.y), ty1 = fmaf(hy, r.inv.y, -r.oinv.y);
-    float tz0 = fmaf(lz, r.inv.z, -r.oinv.z), tz1 = fmaf(hz, r.inv.z, -r.oinv.z);
-    float tn = fmaxf(fmaxf(fminf(tx0, tx1), fminf(ty0, ty1)), fmaxf(fminf(tz0, tz1), tmin));
-    float tf = fminf(fminf(fmaxf(tx0, tx1), fmaxf(ty0, ty1)), fmaxf(tz0, tz1)) * 1.0000004f;
-    tnear = tn;
-    return tn <= fminf(tf, tmax);
 }
 
 // Watertight ray/triangle test.  Products are not contracted into FMAs so
@@ -132,26 +123,27 @@ RTX_DI bool isectSphere(const rtx_sphere &s, V3 o, V3 d, float tmin, float tmax,
 // The two pointers carry their address spaces (3: LDS, 5: private), so that
 // a pop, which reads one or the other, compiles to ds_read and scratch_load
 // rather than to a flat load of a selected pointer.
-typedef __attribute__((address_space(3))) int LdsInt;
-typedef __attribute__((address_space(5))) int PrivInt;
+typedef uint32_t U32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) U32x2 LdsEntry;
+typedef __attribute__((address_space(5))) U32x2 PrivEntry;
 
 template <int BLOCK, int LDS_DEPTH> struct HybridStack {
     static constexpr int kSpill = kStackCapacity - LDS_DEPTH;
-    LdsInt *lds;
-    PrivInt *priv;
+    LdsEntry *lds;
+    PrivEntry *priv;
     int sp;
     // ldsColumn: this thread's column of the block's LDS stack (stride BLOCK);
     // spill: kSpill private entries.
-    RTX_DI void bind(int *ldsColumn, int *spill) {
-        lds = (LdsInt *)ldsColumn;
-        priv = (PrivInt *)spill;
+    RTX_DI void bind(U32x2 *ldsColumn, U32x2 *spill) {
+        lds = (LdsEntry *)ldsColumn;
+        priv = (PrivEntry *)spill;
     }
-    RTX_DI void push(int x) {
+    RTX_DI void push(U32x2 x) {
         if (sp < LDS_DEPTH) lds[sp * BLOCK] = x;
         else priv[sp - LDS_DEPTH] = x;
         sp++;
     }
-    RTX_DI int pop() {
+    RTX_DI U32x2 pop() {
         sp--;
         return sp < LDS_DEPTH ? lds[sp * BLOCK] : priv[sp - LDS_DEPTH];
     }
@@ -159,57 +151,133 @@ template <int BLOCK, int LDS_DEPTH> struct HybridStack {
 
 // Whole stack in a private array (kStackCapacity entries, the caller's).
 struct PrivateStack {
-    PrivInt *priv;
+    PrivEntry *priv;
     int sp;
-    RTX_DI PrivateStack(int *spill) : priv((PrivInt *)spill), sp(0) {}
-    RTX_DI void push(int x) { priv[sp++] = x; }
-    RTX_DI int pop() { return priv[--sp]; }
+    RTX_DI PrivateStack(U32x2 *spill) : priv((PrivEntry *)spill), sp(0) {}
+    RTX_DI void push(U32x2 x) { priv[sp++] = x; }
+    RTX_DI U32x2 pop() { return priv[--sp]; }
 };
 
 struct VisitCount {
     uint32_t nodes = 0, prims = 0;
 };
 
-constexpr int32_t kLinkDone = (int32_t)0x80000000; // no node: a leaf never encodes to this
+// Where a ray is in the tree: the inner children of one node still to visit
+// (group.x their node's childBase, group.y the slots to visit in bits 0-7 and
+// the node's imask in bits 8-15; no bit set: no more nodes), and the leaves of
+// the last node still to test (slots in leaves, the node's triBase and counts)
+// after the triLeft triangles from tri on of the leaf under way.
+struct TravPos {
+    U32x2 group;
+    uint32_t leaves, triBase, counts;
+    uint32_t tri, triLeft;
+    RTX_DI bool atNode() const { return (group.y & 0xFFu) != 0u; }
+    RTX_DI bool atLeaf() const { return (leaves | triLeft) != 0u; }
+};
+// The root, as the only child of a node that is not there.
+RTX_DI void startPos(TravPos &p) {
+    p.group = U32x2{0u, 0x101u};
+    p.leaves = p.triLeft = 0u;
+}
+RTX_DI void endPos(TravPos &p) {
+    p.group.y = 0u;
+    p.leaves = p.triLeft = 0u;
+}
 
-template <class Stack> RTX_DI int popOrDone(Stack &st) { return st.sp == 0 ? kLinkDone : st.pop(); }
+RTX_DI float ubyte(uint32_t w, int k) { return (float)((w >> (8 * k)) & 0xFFu); }
 
-// One four-wide node visit: of the children whose boxes the ray enters within
-// [tmin, tmax], the nearest is returned and the others are pushed, farthest
-// first; with none entered, the next stack entry (kLinkDone when empty).
+// Of a set of slots, the one the ray comes to first.
+RTX_DI int nearSlot(const TravRay &r, uint32_t set) {
+    uint32_t h = set & r.near4;
+    set = h ? h : set;
+    h = set & r.near2;
+    set = h ? h : set;
+    h = set & r.near1;
+    set = h ? h : set;
+    return __ffs(set) - 1;
+}
+
+// The four-wide FP32 nodes before these took seven 16-byte loads and 28
+// visits a ray in the 262,144-triangle room, and the loads' address
+// processing bounded the launch (TA busy 95%, 0.70 cache accesses a cycle and
+// CU).  These take five loads and 19 visits (TA busy 76%); the launch is bound
+// by vector instructions, 48 conversions and 48 FMAs of a visit's 180 first
+// (v_perm pairs into v_fma_mix instead of conversions measured the same):
+// 1.49 -> 0.97 ms for 2 x 1080p paths (1.85 before the rays went out in chunks).
+// One node visit: the next of the group's children in the ray's order is
+// taken (the rest pushed), its children's boxes are tested against
+// [tmin, tmax], and the entered ones become the group and the leaves to test.
+// With no inner child entered the next stack entry becomes the group.
+//
+// A box plane is one FMA, fma(q, 2^e inv, p inv - o inv).  Its error is below
+// (4 |o| + |p| + 2 |l|) 2^-24 in units of |inv| for a plane at l, which the
+// boxes' padding of (|x| + S) 2^-19 covers for rays that start within 7 S of
+// the origin; rays from further away are covered by the factor 1 + 2 gamma_3
+// on the exit distance (Ize, "Robust BVH ray traversal", JCGT 2013).  So a box
+// the exact ray touches is never culled, and the hits do not depend on the
+// tree.  A NaN plane (0 * inf, inf - inf) constrains nothing: min and max
+// return their other operand.
 template <class SceneT, class Stack>
-RTX_DI int nodeStep4(const SceneT &S, const TravRay &r, float tmin, float tmax, int link, Stack &st) {
-    const float4 *np = S.nodes + 8 * (size_t)link;
-    const float4 lx = np[0], hx = np[1], ly = np[2], hy = np[3], lz = np[4], hz = np[5];
-    const int4 ln = *reinterpret_cast<const int4 *>(np + 6);
-    const float inf = __int_as_float(0x7f800000);
-    float t[4], tn;
-    int c[4] = {ln.x, ln.y, ln.z, ln.w};
-    t[0] = slab(lx.x, ly.x, lz.x, hx.x, hy.x, hz.x, r, tmin, tmax, tn) ? tn : inf;
-    t[1] = slab(lx.y, ly.y, lz.y, hx.y, hy.y, hz.y, r, tmin, tmax, tn) ? tn : inf;
-    t[2] = slab(lx.z, ly.z, lz.z, hx.z, hy.z, hz.z, r, tmin, tmax, tn) ? tn : inf;
-    t[3] = slab(lx.w, ly.w, lz.w, hx.w, hy.w, hz.w, r, tmin, tmax, tn) ? tn : inf;
-    // sorting network on (t, link), ascending t
-    auto cs = [&](int i, int j) {
-        if (t[j] < t[i]) {
-            float tt = t[i];
-            t[i] = t[j];
-            t[j] = tt;
-            int cc = c[i];
-            c[i] = c[j];
-            c[j] = cc;
+RTX_DI void nodeStep(const SceneT &S, const TravRay &r, float tmin, float tmax, TravPos &pos, Stack &st) {
+    const int slot = nearSlot(r, pos.group.y & 0xFFu);
+    const uint32_t rank = __popc((pos.group.y >> 8) & ((1u << slot) - 1u));
+    const float4 *np = S.nodes + (size_t)(pos.group.x + rank * kWideNodeSlots);
+    const uint4 n0 = *reinterpret_cast<const uint4 *>(np), n1 = *reinterpret_cast<const uint4 *>(np + 1);
+    const uint4 bx = *reinterpret_cast<const uint4 *>(np + 2), by = *reinterpret_cast<const uint4 *>(np + 3),
+                bz = *reinterpret_cast<const uint4 *>(np + 4);
+    pos.group.y &= ~(1u << slot);
+    if (pos.atNode()) st.push(pos.group);
+    const float sx = __uint_as_float((n0.w & 0xFFu) << 23) * r.inv.x;
+    const float sy = __uint_as_float(((n0.w >> 8) & 0xFFu) << 23) * r.inv.y;
+    const float sz = __uint_as_float(((n0.w >> 16) & 0xFFu) << 23) * r.inv.z;
+    const float ox = fmaf(__uint_as_float(n0.x), r.inv.x, -r.oinv.x);
+    const float oy = fmaf(__uint_as_float(n0.y), r.inv.y, -r.oinv.y);
+    const float oz = fmaf(__uint_as_float(n0.z), r.inv.z, -r.oinv.z);
+    const bool negx = r.near1 == 0xAAu, negy = r.near2 == 0xCCu, negz = r.near4 == 0xF0u;
+    uint32_t miss = 0; // bit 7 - slot
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        const uint32_t lx = half ? bx.y : bx.x, hx = half ? bx.w : bx.z, ly = half ? by.y : by.x,
+                       hy = half ? by.w : by.z, lz = half ? bz.y : bz.x, hz = half ? bz.w : bz.z;
+        const uint32_t nx = negx ? hx : lx, fx = negx ? lx : hx, ny = negy ? hy : ly, fy = negy ? ly : hy,
+                       nz = negz ? hz : lz, fz = negz ? lz : hz;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float tn = fmaxf(fmaxf(fmaxf(fmaf(ubyte(nx, k), sx, ox), fmaf(ubyte(ny, k), sy, oy)),
+                                         fmaf(ubyte(nz, k), sz, oz)),
+                                   tmin);
+            const float tf = fminf(fminf(fminf(fmaf(ubyte(fx, k), sx, ox), fmaf(ubyte(fy, k), sy, oy)),
+                                         fmaf(ubyte(fz, k), sz, oz)),
+                                   tmax);
+            // the sign of exit - entry, shifted into the slots' misses
+            const float in = fmaf(tf, 1.0000004f, -tn);
+            miss = __builtin_amdgcn_alignbit(miss, __float_as_uint(in), 31);
         }
-    };
-    cs(0, 1);
-    cs(2, 3);
-    cs(0, 2);
-    cs(1, 3);
-    cs(1, 2);
-    if (t[3] < inf) st.push(c[3]);
-    if (t[2] < inf) st.push(c[2]);
-    if (t[1] < inf) st.push(c[1]);
-    if (t[0] < inf) return c[0];
-    return popOrDone(st);
+    }
+    const uint32_t imask = n0.w >> 24;
+    const uint32_t hits = (__brev(~miss) >> 24) & (n1.w & 0xFFu);
+    pos.leaves = hits & ~imask;
+    pos.triBase = n1.y;
+    pos.counts = n1.z;
+    pos.group = U32x2{n1.x, (hits & imask) | (imask << 8)};
+    if (!pos.atNode() && st.sp != 0) pos.group = st.pop();
+}
+
+// The next triangle to test (in 16-byte units), at a leaf.
+RTX_DI uint32_t nextTri(TravPos &pos) {
+    if (pos.triLeft == 0u) {
+        const int shift = 4 * (__ffs(pos.leaves) - 1);
+        pos.leaves &= pos.leaves - 1u;
+        const uint32_t below = pos.counts & ((1u << shift) - 1u);
+        // the nibbles' sum: at most 7 x 15
+        const uint32_t sum = (((below & 0x0F0F0F0Fu) + ((below >> 4) & 0x0F0F0F0Fu)) * 0x01010101u) >> 24;
+        pos.tri = pos.triBase + 3u * sum;
+        pos.triLeft = (pos.counts >> shift) & 15u;
+    }
+    const uint32_t t = pos.tri;
+    pos.tri += 3u;
+    pos.triLeft--;
+    return t;
 }
 
 // Closest hit (ANY = false) or first hit (ANY = true) in [tmin, tmax].
@@ -233,37 +301,29 @@ RTX_DI int traverse(const DevScene &S, const TravRay &r, float tmin, float &tmax
         }
     }
     st.sp = 0;
-    int link = 0;
-    for (;;) {
-        if (link >= 0) {
-            if (COUNT) vc.nodes++;
-            link = nodeStep4(S, r, tmin, tmax, link, st);
-            if (link == kLinkDone) break;
-        } else {
-            uint32_t leaf = ~(uint32_t)link;
-            uint32_t start = leaf >> 4, cnt = (leaf & 15u) + 1u;
-            const float4 *tp = S.tris + 3 * (size_t)start;
-            for (uint32_t k = 0; k < cnt; ++k) {
-                float4 v0 = tp[3 * k], v1 = tp[3 * k + 1], v2 = tp[3 * k + 2];
-                if (COUNT) vc.prims++;
-                float t, u, v;
-                if (isectTri(r, v0, v1, v2, tmin, tmax, t, u, v)) {
-                    int id = __float_as_int(v0.w);
-                    if (id & kAlphaBit) {
-                        id &= ~kAlphaBit;
-                        if (!alphaAccept(S, id, r.o.x, t, u, v, randomUInt)) continue;
-                    }
-                    if (ANY) return id;
-                    if (best < 0 || t < tmax || id < best) {
-                        tmax = t;
-                        best = id;
-                        bu = u;
-                        bv = v;
-                    }
+    TravPos pos;
+    startPos(pos);
+    while (pos.atNode()) {
+        if (COUNT) vc.nodes++;
+        nodeStep(S, r, tmin, tmax, pos, st);
+        while (pos.atLeaf()) {
+            const float4 *tp = S.tris + (size_t)nextTri(pos);
+            if (COUNT) vc.prims++;
+            float t, u, v;
+            if (isectTri(r, tp[0], tp[1], tp[2], tmin, tmax, t, u, v)) {
+                int id = __float_as_int(tp[0].w);
+                if (id & kAlphaBit) {
+                    id &= ~kAlphaBit;
+                    if (!alphaAccept(S, id, r.o.x, t, u, v, randomUInt)) continue;
+                }
+                if (ANY) return id;
+                if (best < 0 || t < tmax || id < best) {
+                    tmax = t;
+                    best = id;
+                    bu = u;
+                    bv = v;
                 }
             }
-            if (st.sp == 0) break;
-            link = st.pop();
         }
     }
     return best;
@@ -294,15 +354,14 @@ RTX_DI bool alphaAccept(const LaneScene &S, int prim, float ox, float t, float b
 // ------------------------------------------------------------------
 // Persistent traversal with lane refill (Aila & Laine 2009, sections 4-5):
 // each wave loops until the queue is drained; lanes whose ray finished
-// fetch a new ray, and node visits and leaf tests alternate with postponed
-// leaves: a lane that reaches a leaf parks it and keeps descending until
-// enough of the wave's lanes wait at a leaf, then those are intersected
-// together.
+// fetch a new ray, and node visits and leaf tests alternate: a lane that
+// enters leaves waits until enough of the wave's lanes do, then those
+// intersect a leaf each together.
 struct LaneRay {
     TravRay r;
     float tmin, tmax, bu, bv;
     int best;
-    int link, leaf;
+    TravPos pos;
     uint32_t idx;
     uint32_t randomUInt; // the frame's, for the any-hit alpha test
     bool any;            // kHitLane: this lane's ray wants any hit
@@ -313,43 +372,30 @@ struct LaneRay {
 // closest-hit rays side by side.
 constexpr int kHitClosest = 0, kHitAny = 1, kHitLane = 2;
 
-// One inner-node visit: returns the next link (pushing the farther entered
-// children), or the next stack entry / kLinkDone when none is entered.
-template <bool COUNT, class SceneT, class Stack>
-RTX_DI int innerStep(const SceneT &S, LaneRay &L, Stack &st, VisitCount &vc) {
-    if (COUNT) vc.nodes++;
-    return nodeStep4(S, L.r, L.tmin, L.tmax, L.link, st);
-}
-
-// Intersects the primitives of leaf link `leaf`; returns true when an any-hit
-// ray is done.
+// Intersects the lane's next triangle; returns true when an any-hit ray is
+// done.
 template <int HIT, bool COUNT, bool ALPHA, class SceneT>
-RTX_DI bool leafStep(const SceneT &S, LaneRay &L, int leaf, VisitCount &vc) {
+RTX_DI bool triStep(const SceneT &S, LaneRay &L, VisitCount &vc) {
     const bool ANY = HIT == kHitAny || (HIT == kHitLane && L.any);
-    uint32_t data = ~(uint32_t)leaf;
-    uint32_t start = data >> 4, cnt = (data & 15u) + 1u;
-    const float4 *tp = S.tris + 3 * (size_t)start;
-    for (uint32_t k = 0; k < cnt; ++k) {
-        float4 v0 = tp[3 * k], v1 = tp[3 * k + 1], v2 = tp[3 * k + 2];
-        if (COUNT) vc.prims++;
-        float t, u, v;
-        if (isectTri(L.r, v0, v1, v2, L.tmin, L.tmax, t, u, v)) {
-            int id = __float_as_int(v0.w);
-            if (ALPHA && (id & kAlphaBit)) {
-                id &= ~kAlphaBit;
-                if (!alphaAccept(S, id, L.r.o.x, t, u, v, L.randomUInt)) continue;
-            }
-            if (ANY) {
-                L.best = id;
-                return true;
-            }
-            if (L.best < 0 || t < L.tmax || id < L.best) {
-                L.tmax = t;
-                L.best = id;
-                L.bu = u;
-                L.bv = v;
-            }
-        }
+    const float4 *tp = S.tris + (size_t)nextTri(L.pos);
+    const float4 v0 = tp[0], v1 = tp[1], v2 = tp[2];
+    if (COUNT) vc.prims++;
+    float t, u, v;
+    if (!isectTri(L.r, v0, v1, v2, L.tmin, L.tmax, t, u, v)) return false;
+    int id = __float_as_int(v0.w);
+    if (ALPHA && (id & kAlphaBit)) {
+        id &= ~kAlphaBit;
+        if (!alphaAccept(S, id, L.r.o.x, t, u, v, L.randomUInt)) return false;
+    }
+    if (ANY) {
+        L.best = id;
+        return true;
+    }
+    if (L.best < 0 || t < L.tmax || id < L.best) {
+        L.tmax = t;
+        L.best = id;
+        L.bu = u;
+        L.bv = v;
     }
     return false;
 }
@@ -359,8 +405,7 @@ template <int HIT, class SceneT> RTX_DI void beginRay(const SceneT &S, LaneRay &
     const bool ANY = HIT == kHitAny || (HIT == kHitLane && L.any);
     L.best = -1;
     L.bu = L.bv = 0.0f;
-    L.link = 0;
-    L.leaf = kLinkDone;
+    startPos(L.pos);
     for (uint32_t i = 0; i < S.numSpheres; ++i) {
         float t;
         if (isectSphere(S.spheres[i], L.r.o, L.r.d, L.tmin, L.tmax, t)) {
@@ -370,7 +415,7 @@ template <int HIT, class SceneT> RTX_DI void beginRay(const SceneT &S, LaneRay &
                 L.best = id;
             }
             if (ANY) {
-                L.link = kLinkDone;
+                endPos(L.pos);
                 return;
             }
         }
@@ -410,17 +455,17 @@ constexpr int kRefillLanes = 24;          // 16 to 32: within 0.3% of each other
 constexpr uint32_t kChunksPerWave = 8, kChunkMax = 512;
 constexpr uint32_t kSpread = 2;
 // Inner nodes are visited while at least kNodeNum / kNodeDen of the active
-// lanes have one to visit; then every lane that holds a leaf intersects it.
-// A ray visits some ten inner nodes a leaf, so waiting until every lane holds
-// a leaf left two thirds of the lanes idle.  1/2 measured the same, 7/8 1-2%
-// slower (more leaf passes over few lanes).
+// lanes have one to visit; then every lane at a leaf intersects that leaf.
+// A ray visits some four inner nodes a leaf, so waiting until every lane is at
+// a leaf left two thirds of the lanes idle.  2/3 measured the same, 1/2 and
+// 7/8 1-2% slower; so did one triangle a lane and pass instead of one leaf.
 constexpr int kNodeNum = 3, kNodeDen = 4;
 
 template <int HIT, bool COUNT, bool ALPHA, class SceneT, class Stack, class Load, class Store>
 RTX_DI void persistentTrace(const SceneT &S, uint32_t n, uint32_t *fetch, Stack &st, VisitCount &vc, Load load,
                             Store store) {
     LaneRay L;
-    L.link = L.leaf = kLinkDone;
+    endPos(L.pos);
     L.idx = 0;
     L.any = HIT == kHitAny;
     bool active = false;
@@ -478,29 +523,19 @@ RTX_DI void persistentTrace(const SceneT &S, uint32_t n, uint32_t *fetch, Stack 
         // inner nodes while most of the active lanes have one to visit
         int nNode;
         do {
-            if (L.link >= 0) {
-                L.link = innerStep<COUNT>(S, L, st, vc);
-                if (L.link < 0 && L.link != kLinkDone && L.leaf == kLinkDone) {
-                    L.leaf = L.link;
-                    L.link = popOrDone(st);
-                }
+            if (!L.pos.atLeaf() && L.pos.atNode()) {
+                if (COUNT) vc.nodes++;
+                nodeStep(S, L.r, L.tmin, L.tmax, L.pos, st);
             }
-            nNode = __popcll(__ballot(L.link >= 0));
+            nNode = __popcll(__ballot(!L.pos.atLeaf() && L.pos.atNode()));
         } while (nNode * kNodeDen >= nActive * kNodeNum && nNode > 0);
-        // one leaf of every lane that holds one
-        if (L.leaf != kLinkDone) {
-            if (leafStep<HIT, COUNT, ALPHA>(S, L, L.leaf, vc)) {
-                L.link = kLinkDone;
-                L.leaf = kLinkDone;
-            } else {
-                L.leaf = kLinkDone;
-                if (L.link < 0 && L.link != kLinkDone) {
-                    L.leaf = L.link;
-                    L.link = popOrDone(st);
-                }
-            }
+        // the next leaf of every lane at one
+        if (L.pos.atLeaf()) {
+            do {
+                if (triStep<HIT, COUNT, ALPHA>(S, L, vc)) endPos(L.pos);
+            } while (L.pos.triLeft != 0u);
         }
-        if (active && L.link == kLinkDone && L.leaf == kLinkDone) {
+        if (active && !L.pos.atLeaf() && !L.pos.atNode()) {
             store(L);
             active = false;
         }

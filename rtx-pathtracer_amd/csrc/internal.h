@@ -15,7 +15,7 @@ namespace rtx {
 
 // ----------------------------------------------------------- device scene
 struct DevScene {
-    const float4 *nodes;      // 8 x float4 per Bvh4Node
+    const float4 *nodes;      // kWideNodeSlots x float4 per Bvh8Node
     const float4 *tris;       // 3 x float4 per triangle in leaf order: v0 (w = prim id bits), v1, v2
     const int4 *triRef;       // per global triangle id: (instance, global indices of its three vertices)
     const rtx_vertex *vertices;
@@ -350,7 +350,7 @@ void launchGenerate(hipStream_t s, const FrameConst *fc, BatchDesc b, PathBuffer
 // extend[esel]), then the probe and shadow queues; fetch[1] must be zero.
 // poll (may be NULL): host-visible slot for the bounce's starting queue
 // lengths (extend, probe, shadow, done), written by the first thread
-// ldsEntries: stack entries per thread in LDS, 12, 16, 20 or 24
+// ldsEntries: 4-byte stack words per thread in LDS, 12, 16, 20 or 24
 void launchTraceP(hipStream_t s, const DevScene &S, Queue qe, int esel, Queue qs, Queue qp, PathBuffers pb,
                   Counters *cnt, uint32_t *poll, bool countVisits, int blocks, int ldsEntries);
 // the two ray queries (closest hit / occlusion); *fetch must be zero

@@ -23,7 +23,8 @@
 namespace rtx {
 
 constexpr int kTraceBlock = 128;
-constexpr int kLdsStack = 20;
+constexpr int kTraceWaves = 7; // per SIMD: at most 72 VGPRs (six waves and the 79 the compiler would take: 2% slower)
+constexpr int kLdsStack = 20; // 4-byte words: two a stack entry
 constexpr int kShadeBlock = 256;
 
 // --------------------------------------------------------- wave helpers
@@ -403,7 +404,7 @@ RTX_DI int nearestLight(const DevScene &S, V3 o, V3 d, float tmin, float &tHit, 
 // with it (kTracePA), so that the test's code stays out of the common loop.
 template <bool COUNT, bool ALPHA, int LDS>
 RTX_DI void traceBody(const DevScene &S, const Queue &qe, int esel, const Queue &qs, const Queue &qp,
-                      const PathBuffers &pb, Counters *cnt, uint32_t *poll, int *stackMem) {
+                      const PathBuffers &pb, Counters *cnt, uint32_t *poll, U32x2 *stackMem) {
     const uint32_t ne = cnt->extend[esel], np = cnt->probe, ns = cnt->shadow;
     const uint32_t nep = ne + np;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -416,8 +417,8 @@ RTX_DI void traceBody(const DevScene &S, const Queue &qe, int esel, const Queue 
         cnt->extend[esel ^ 1] = 0;
         cnt->done[esel] = 0;
     }
-    HybridStack<kTraceBlock, LDS> st;
-    int spill[HybridStack<kTraceBlock, LDS>::kSpill];
+    HybridStack<kTraceBlock, LDS / 2> st;
+    U32x2 spill[HybridStack<kTraceBlock, LDS / 2>::kSpill];
     st.bind(stackMem + threadIdx.x, spill);
     VisitCount vc, vk[3];
     // the queues' arrays as plain pointers, read in per-queue branches (a
@@ -489,19 +490,19 @@ RTX_DI void traceBody(const DevScene &S, const Queue &qe, int esel, const Queue 
     flushVisits<COUNT>(vk[1], cnt, 1);
     flushVisits<COUNT>(vk[2], cnt, 2);
 }
-// LDS: stack entries per thread held in LDS (the rest in scratch), a
-// launch-shape choice (rtx_tuning.ldsStackEntries): more entries cost LDS and
-// so resident blocks.
+// LDS: 4-byte words of the stack per thread held in LDS (the rest in scratch;
+// an entry takes two), a launch-shape choice (rtx_tuning.ldsStackEntries):
+// more cost LDS and so resident blocks.
 template <bool COUNT, int LDS = kLdsStack>
-__global__ __launch_bounds__(kTraceBlock) void kTraceP(DevScene S, Queue qe, int esel, Queue qs, Queue qp,
+__global__ __launch_bounds__(kTraceBlock, kTraceWaves) void kTraceP(DevScene S, Queue qe, int esel, Queue qs, Queue qp,
                                                       PathBuffers pb, Counters *cnt, uint32_t *poll) {
-    __shared__ int stackMem[LDS * kTraceBlock];
+    __shared__ U32x2 stackMem[LDS / 2 * kTraceBlock];
     traceBody<COUNT, false, LDS>(S, qe, esel, qs, qp, pb, cnt, poll, stackMem);
 }
 template <bool COUNT, int LDS = kLdsStack>
-__global__ __launch_bounds__(kTraceBlock) void kTracePA(DevScene S, Queue qe, int esel, Queue qs, Queue qp,
+__global__ __launch_bounds__(kTraceBlock, kTraceWaves) void kTracePA(DevScene S, Queue qe, int esel, Queue qs, Queue qp,
                                                        PathBuffers pb, Counters *cnt, uint32_t *poll) {
-    __shared__ int stackMem[LDS * kTraceBlock];
+    __shared__ U32x2 stackMem[LDS / 2 * kTraceBlock];
     traceBody<COUNT, true, LDS>(S, qe, esel, qs, qp, pb, cnt, poll, stackMem);
 }
 
@@ -512,9 +513,9 @@ __global__ __launch_bounds__(kTraceBlock) void kTracePA(DevScene S, Queue qe, in
 // copies every slot's live-path count after the bounce's queue lengths into
 // the host-visible slot `poll` (4 + numSlots words).
 template <bool ALPHA>
-__global__ __launch_bounds__(kTraceBlock) void kTraceM(MultiArgs ma, Queue qe, int esel, Queue qs, Queue qp,
+__global__ __launch_bounds__(kTraceBlock, kTraceWaves) void kTraceM(MultiArgs ma, Queue qe, int esel, Queue qs, Queue qp,
                                                       PathBuffers pb, Counters *cnt, uint32_t *poll) {
-    __shared__ int stackMem[kLdsStack * kTraceBlock];
+    __shared__ U32x2 stackMem[kLdsStack / 2 * kTraceBlock];
     const uint32_t ne = cnt->extend[esel], np = cnt->probe, ns = cnt->shadow;
     const uint32_t nep = ne + np;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -529,8 +530,8 @@ __global__ __launch_bounds__(kTraceBlock) void kTraceM(MultiArgs ma, Queue qe, i
     }
     if (blockIdx.x == 0 && poll)
         for (uint32_t k = threadIdx.x; k < ma.numSlots; k += kTraceBlock) poll[4 + k] = ma.slotAlive[k];
-    HybridStack<kTraceBlock, kLdsStack> st;
-    int spill[HybridStack<kTraceBlock, kLdsStack>::kSpill];
+    HybridStack<kTraceBlock, kLdsStack / 2> st;
+    U32x2 spill[HybridStack<kTraceBlock, kLdsStack / 2>::kSpill];
     st.bind(stackMem + threadIdx.x, spill);
     VisitCount vc;
     LaneScene ls{};
@@ -964,7 +965,7 @@ RTX_DI void shadeLane(const DevScene &S, const DevIC &IC, const DevGuiding &G, c
                         // The reference returns from NEE here if the shadow ray is
                         // unoccluded (raytrace.rgen:653-655), skipping the probe's draws:
                         // resolve visibility now to keep the random stream in step.
-                        int spill[kStackCapacity];
+                        U32x2 spill[kStackCapacity];
                         PrivateStack ps(spill);
                         VisitCount vc0;
                         TravRay sr = makeTravRay(h.worldPos, lightDir);
@@ -1394,11 +1395,11 @@ __global__ __launch_bounds__(256) void kResolveImage(const float4 *accum, uint32
 // The two ray queries (closest hit, occlusion) with the persistent lane-refill
 // traversal of the wavefront.
 template <bool ANY>
-__global__ __launch_bounds__(kTraceBlock) void kQueryP(DevScene S, const rtx_ray *rays, uint32_t n, void *out,
+__global__ __launch_bounds__(kTraceBlock, kTraceWaves) void kQueryP(DevScene S, const rtx_ray *rays, uint32_t n, void *out,
                                                       uint32_t *fetch) {
-    __shared__ int stackMem[kLdsStack * kTraceBlock];
-    HybridStack<kTraceBlock, kLdsStack> st;
-    int spill[HybridStack<kTraceBlock, kLdsStack>::kSpill];
+    __shared__ U32x2 stackMem[kLdsStack / 2 * kTraceBlock];
+    HybridStack<kTraceBlock, kLdsStack / 2> st;
+    U32x2 spill[HybridStack<kTraceBlock, kLdsStack / 2>::kSpill];
     st.bind(stackMem + threadIdx.x, spill);
     VisitCount vc;
     persistentTrace<ANY ? kHitAny : kHitClosest, false, true>( // alpha-tested triangles with randomUInt 0
