@@ -59,6 +59,21 @@ RTX_DI void waveAppend2(bool a, uint32_t *ca, bool b, uint32_t *cb, int &ia, int
     ib = b ? (int)(baseb + (uint32_t)__popcll(mb & below)) : -1;
 }
 
+// One append of both the `a` and the `b` lanes, the b lanes behind the a
+// lanes: one atomic.
+RTX_DI void waveAppendBoth(bool a, bool b, uint32_t *counter, int &ia, int &ib) {
+    const uint64_t ma = __ballot(a), mb = __ballot(b);
+    const int lane = (int)__lane_id();
+    const uint32_t na = (uint32_t)__popcll(ma), nb = (uint32_t)__popcll(mb);
+    const int leader = (ma | mb) ? __ffsll((unsigned long long)(ma | mb)) - 1 : 0;
+    uint32_t base = 0;
+    if ((ma | mb) && lane == leader) base = atomicAdd(counter, na + nb);
+    base = __shfl(base, leader);
+    const uint64_t below = lane == 0 ? 0ull : ((~0ull) >> (64 - lane));
+    ia = a ? (int)(base + (uint32_t)__popcll(ma & below)) : -1;
+    ib = b ? (int)(base + na + (uint32_t)__popcll(mb & below)) : -1;
+}
+
 // Runs body(k) once for every distinct value k of `key` among the lanes
 // with `active`, with exactly the lanes holding that key active and k
 // wave-uniform (read with readlane, so per-key data are scalar loads).  The
@@ -178,7 +193,7 @@ __global__ __launch_bounds__(256) void kGenerate(const FrameConst *__restrict__ 
     const FrameConst &fc = *fcp;
     uint32_t pid = blockIdx.x * 256 + threadIdx.x;
     if (pid == 0) {
-        cnt->extend[qsel] = b.numPaths;
+        cnt->extend[qsel].v = b.numPaths;
         if (fc.nrc) *pb.nrcQueryCount = 0u;
     }
     const bool active = pid < b.numPaths;
@@ -249,7 +264,7 @@ __global__ __launch_bounds__(256) void kGenerateM(const SlotDesc *__restrict__ s
         pb.thr[pid] = make_float4(1.0f, 1.0f, 1.0f, __uint_as_float(kFlagsCameraStart));
         pb.result[pid] = make_float4(0.0f, 0.0f, 0.0f, kTMax);
     }
-    const int qi = waveAppend(active, &cnt->extend[qsel]);
+    const int qi = waveAppend(active, &cnt->extend[qsel].v);
     if (active) {
         q0.id[qi] = (int)pid;
         q0.org[qi] = f4(o, kTMin);
@@ -259,11 +274,11 @@ __global__ __launch_bounds__(256) void kGenerateM(const SlotDesc *__restrict__ s
 
 // Writes slot `slot`'s descriptor and its live-path count (the batch's
 // paths); passed by value so that the host's copy needs no lifetime.
-__global__ __launch_bounds__(256) void kInstallSlot(SlotDesc sd, SlotDesc *slots, uint32_t slot, uint32_t *alive) {
+__global__ __launch_bounds__(256) void kInstallSlot(SlotDesc sd, SlotDesc *slots, uint32_t slot, CounterWord *alive) {
     const uint32_t *src = reinterpret_cast<const uint32_t *>(&sd);
     uint32_t *dst = reinterpret_cast<uint32_t *>(slots + slot);
     for (uint32_t k = threadIdx.x; k < sizeof(SlotDesc) / 4; k += 256) dst[k] = src[k];
-    if (threadIdx.x == 0) alive[slot] = sd.b.numPaths;
+    if (threadIdx.x == 0) alive[slot].v = sd.b.numPaths;
 }
 
 // The sub-paths of calculateCacheData (raytrace.rgen:1246-1263) for jobs
@@ -284,7 +299,7 @@ __global__ __launch_bounds__(256) void kGenerateIC(IcBuffers ic, uint32_t frameS
         numPaths = min(numPaths, (jEnd > j0 ? jEnd - j0 : 0u) * (uint32_t)kIcStrata);
     }
     const uint32_t local = blockIdx.x * 256 + threadIdx.x;
-    if (local == 0) cnt->extend[qsel] = qBase + numPaths; // after the qBase entries already queued
+    if (local == 0) cnt->extend[qsel].v = qBase + numPaths; // after the qBase entries already queued
     if (local >= numPaths) return;
     const uint32_t pid = pidBase + local, qi = qBase + local;
     const uint32_t job = j0 + local / kIcStrata, st = local % kIcStrata;
@@ -397,7 +412,7 @@ RTX_DI int nearestLight(const DevScene &S, V3 o, V3 d, float tmin, float &tHit, 
 // pendShadow).  Ray i of the launch is extend ray i for i < ne, probe ray
 // i - ne below ne + np, shadow ray i - ne - np after that.  The closest-hit
 // rays come first so that the launch's tail is made of short occlusion rays,
-// and a bounce pays one launch and one tail.  Work counter: fetch[1].
+// and a bounce pays one launch and one tail.  Work counter: fetch.
 // COUNT builds count node and triangle visits per queue (visit kinds 0
 // extend, 1 shadow, 2 probe).  The kernels come in two builds: without the
 // any-hit alpha test (scenes with no textured triangles, the hot path) and
@@ -405,17 +420,17 @@ RTX_DI int nearestLight(const DevScene &S, V3 o, V3 d, float tmin, float &tHit, 
 template <bool COUNT, bool ALPHA, int LDS>
 RTX_DI void traceBody(const DevScene &S, const Queue &qe, int esel, const Queue &qs, const Queue &qp,
                       const PathBuffers &pb, Counters *cnt, uint32_t *poll, U32x2 *stackMem) {
-    const uint32_t ne = cnt->extend[esel], np = cnt->probe, ns = cnt->shadow;
+    const uint32_t ne = cnt->extend[esel].v, np = cnt->probe.v, ns = cnt->shadow.v;
     const uint32_t nep = ne + np;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         atomicAdd(&cnt->extendRays, (unsigned long long)ne);
         atomicAdd(&cnt->probeRays, (unsigned long long)np);
         atomicAdd(&cnt->shadowRays, (unsigned long long)ns);
-        reportBounce(poll, ne, np, ns, cnt->done[esel ^ 1]);
+        reportBounce(poll, ne, np, ns, cnt->done[esel ^ 1].v);
         // the lists the bounce's kFinish and kShade append to: their previous
         // contents (two bounces back) are consumed
-        cnt->extend[esel ^ 1] = 0;
-        cnt->done[esel] = 0;
+        cnt->extend[esel ^ 1].v = 0;
+        cnt->done[esel].v = 0;
     }
     HybridStack<kTraceBlock, LDS / 2> st;
     U32x2 spill[HybridStack<kTraceBlock, LDS / 2>::kSpill];
@@ -430,7 +445,7 @@ RTX_DI void traceBody(const DevScene &S, const Queue &qe, int esel, const Queue 
     const uint32_t *pathSeed = qe.pathSeed;
     const uint32_t secDiv = qs.seedDiv; // probe and shadow entries: path * numNEE + j
     persistentTrace<kHitLane, COUNT, ALPHA>(
-        S, nep + ns, &cnt->fetch[1], st, vc,
+        S, nep + ns, &cnt->fetch.v, st, vc,
         [&](uint32_t i, LaneRay &L) {
             const bool ext = i < ne, shadow = i >= nep;
             const uint32_t j = ext ? i : shadow ? i - nep : i - ne;
@@ -516,20 +531,20 @@ template <bool ALPHA>
 __global__ __launch_bounds__(kTraceBlock, kTraceWaves) void kTraceM(MultiArgs ma, Queue qe, int esel, Queue qs, Queue qp,
                                                       PathBuffers pb, Counters *cnt, uint32_t *poll) {
     __shared__ U32x2 stackMem[kLdsStack / 2 * kTraceBlock];
-    const uint32_t ne = cnt->extend[esel], np = cnt->probe, ns = cnt->shadow;
+    const uint32_t ne = cnt->extend[esel].v, np = cnt->probe.v, ns = cnt->shadow.v;
     const uint32_t nep = ne + np;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         atomicAdd(&cnt->extendRays, (unsigned long long)ne);
         atomicAdd(&cnt->probeRays, (unsigned long long)np);
         atomicAdd(&cnt->shadowRays, (unsigned long long)ns);
-        reportBounce(poll, ne, np, ns, cnt->done[esel ^ 1]);
+        reportBounce(poll, ne, np, ns, cnt->done[esel ^ 1].v);
         // the lists the bounce's kFinish and kShade append to: their previous
         // contents (two bounces back) are consumed
-        cnt->extend[esel ^ 1] = 0;
-        cnt->done[esel] = 0;
+        cnt->extend[esel ^ 1].v = 0;
+        cnt->done[esel].v = 0;
     }
     if (blockIdx.x == 0 && poll)
-        for (uint32_t k = threadIdx.x; k < ma.numSlots; k += kTraceBlock) poll[4 + k] = ma.slotAlive[k];
+        for (uint32_t k = threadIdx.x; k < ma.numSlots; k += kTraceBlock) poll[4 + k] = ma.slotAlive[k].v;
     HybridStack<kTraceBlock, kLdsStack / 2> st;
     U32x2 spill[HybridStack<kTraceBlock, kLdsStack / 2>::kSpill];
     st.bind(stackMem + threadIdx.x, spill);
@@ -541,7 +556,7 @@ __global__ __launch_bounds__(kTraceBlock, kTraceWaves) void kTraceM(MultiArgs ma
     float4 *pendShadow = pb.pendShadow, *pendProbe = pb.pendProbe;
     const uint32_t *frameSeed = pb.frameSeed;
     persistentTrace<kHitLane, false, ALPHA>(
-        ls, nep + ns, &cnt->fetch[1], st, vc,
+        ls, nep + ns, &cnt->fetch.v, st, vc,
         [&](uint32_t i, LaneRay &L) {
             const bool ext = i < ne, shadow = i >= nep;
             const uint32_t j = ext ? i : shadow ? i - nep : i - ne;
@@ -593,7 +608,7 @@ __global__ __launch_bounds__(kTraceBlock, kTraceWaves) void kTraceM(MultiArgs ma
 // emitter first never enter this queue).
 __global__ __launch_bounds__(256) void kProbeResolve(DevScene S, const FrameConst *__restrict__ fcp, Queue q,
                                                      PathBuffers pb, Counters *cnt, int qsel) {
-    const uint32_t n = cnt->probe;
+    const uint32_t n = cnt->probe.v;
     const bool power = fcp->pc.usePowerHeuristic != 0;
     for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
         float4 o4 = q.org[i], d4 = q.dir[i], base = q.aux[i], hit = q.hit[i];
@@ -607,7 +622,7 @@ __global__ __launch_bounds__(256) void kProbeResolve(DevScene S, const FrameCons
 // The same over the serving pool: probe entry ids are NEE slots, path * neeStride + j.
 __global__ __launch_bounds__(256) void kProbeResolveM(MultiArgs ma, Queue q, PathBuffers pb, Counters *cnt,
                                                       int qsel) {
-    const uint32_t n = cnt->probe;
+    const uint32_t n = cnt->probe.v;
     for (uint32_t base = blockIdx.x * 256; base < n; base += gridDim.x * 256) {
         const uint32_t i = base + threadIdx.x;
         const bool active = i < n;
@@ -720,7 +735,7 @@ RTX_DI void shadeLane(const DevScene &S, const DevIC &IC, const DevGuiding &G, c
     gp.on = fc.pc.useGuiding != 0;
     gp.parallax = fc.pc.useParallaxCompensation != 0;
     gp.prob = fc.pc.guidingProb;
-    uint32_t *nextCount = &cnt->extend[qsel ^ 1];
+    uint32_t *nextCount = &cnt->extend[qsel ^ 1].v;
     bool cont = false, isDone = false, doNee = false;
     uint32_t pid = 0;
     Rng rng{0};
@@ -1012,15 +1027,15 @@ RTX_DI void shadeLane(const DevScene &S, const DevIC &IC, const DevGuiding &G, c
                 }
             }
         }
-        int si, pi;
-        waveAppend2(wantShadow, &cnt->shadow, wantProbe, &cnt->probe, si, pi);
-        if (lightFirst) {
-            const int oi = waveAppend(wantOcc, &cnt->shadow);
-            if (wantOcc) {
-                qs.id[oi] = (int)slot | kProbeOccBit;
-                qs.org[oi] = f4(h.worldPos, kTMin);
-                qs.dir[oi] = f4(bsdfDir, occMax);
-            }
+        // a light-first probe's occlusion ray goes to the shadow queue, behind
+        // the wave's shadow rays; the other scenes' probes to their own
+        int si, pi = -1, oi = -1;
+        if (lightFirst) waveAppendBoth(wantShadow, wantOcc, &cnt->shadow.v, si, oi);
+        else waveAppend2(wantShadow, &cnt->shadow.v, wantProbe, &cnt->probe.v, si, pi);
+        if (wantOcc) {
+            qs.id[oi] = (int)slot | kProbeOccBit;
+            qs.org[oi] = f4(h.worldPos, kTMin);
+            qs.dir[oi] = f4(bsdfDir, occMax);
         }
         if (wantShadow) {
             qs.id[si] = (int)slot;
@@ -1131,7 +1146,7 @@ RTX_DI void shadeLane(const DevScene &S, const DevIC &IC, const DevGuiding &G, c
         }
     }
     int qi, di;
-    waveAppend2(cont, nextCount, isDone, &cnt->done[qsel], qi, di);
+    waveAppend2(cont, nextCount, isDone, &cnt->done[qsel].v, qi, di);
     if (cont) {
         qout.id[qi] = (int)pid;
         qout.org[qi] = f4(h.worldPos, kTMin);
@@ -1144,7 +1159,7 @@ __global__ __launch_bounds__(kShadeBlock, 2) void kShade(DevScene S, DevIC IC, D
                                                       const FrameConst *__restrict__ fcp, BatchDesc b, PathBuffers pb,
                                                       Queue qin, Queue qout, Queue qs, Queue qp, int32_t *done,
                                                       Counters *cnt, int qsel) {
-    const uint32_t n = cnt->extend[qsel];
+    const uint32_t n = cnt->extend[qsel].v;
     for (uint32_t base = blockIdx.x * kShadeBlock; base < n; base += gridDim.x * kShadeBlock) {
         const uint32_t i = base + threadIdx.x;
         shadeLane(S, IC, G, *fcp, b, pb, qin, qout, qs, qp, done, cnt, qsel, i, i < n);
@@ -1159,7 +1174,7 @@ __global__ __launch_bounds__(kShadeBlock, 2) void kShade2(DevScene S, DevIC IC, 
                                                        const FrameConst *__restrict__ fcp2, BatchDesc b2,
                                                        uint32_t split, PathBuffers pb, Queue qin, Queue qout,
                                                        Queue qs, Queue qp, int32_t *done, Counters *cnt, int qsel) {
-    const uint32_t n = cnt->extend[qsel];
+    const uint32_t n = cnt->extend[qsel].v;
     for (uint32_t base = blockIdx.x * kShadeBlock; base < n; base += gridDim.x * kShadeBlock) {
         const uint32_t i = base + threadIdx.x;
         const bool active = i < n;
@@ -1177,7 +1192,7 @@ __global__ __launch_bounds__(kShadeBlock, 2) void kShade2(DevScene S, DevIC IC, 
 // single-job kernel.
 __global__ __launch_bounds__(kShadeBlock, 2) void kShadeM(MultiArgs ma, PathBuffers pb, Queue qin, Queue qout,
                                                        Queue qs, Queue qp, int32_t *done, Counters *cnt, int qsel) {
-    const uint32_t n = cnt->extend[qsel];
+    const uint32_t n = cnt->extend[qsel].v;
     for (uint32_t base = blockIdx.x * kShadeBlock; base < n; base += gridDim.x * kShadeBlock) {
         const uint32_t i = base + threadIdx.x;
         const bool active = i < n;
@@ -1205,7 +1220,7 @@ RTX_DI bool finishLane(const FrameConst &fc, const BatchDesc &b, const PathBuffe
     const uint32_t numNEE = fc.numNEE;
     const bool record = fc.record != 0;
     const bool segments = fc.segments != 0;
-    uint32_t *nextCount = &cnt->extend[qsel ^ 1];
+    uint32_t *nextCount = &cnt->extend[qsel ^ 1].v;
     bool again = false, splitNext = false;
     uint32_t pid = 0;
     V3 o = v3(0.0f), dir = v3(0.0f, 0.0f, 1.0f);
@@ -1292,15 +1307,15 @@ RTX_DI bool finishLane(const FrameConst &fc, const BatchDesc &b, const PathBuffe
 // kShade refills them.
 RTX_DI void finishClears(Counters *cnt) {
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        cnt->shadow = 0;
-        cnt->probe = 0;
-        cnt->fetch[0] = cnt->fetch[1] = cnt->fetch[2] = 0;
+        cnt->shadow.v = 0;
+        cnt->probe.v = 0;
+        cnt->fetch.v = 0;
     }
 }
 
 __global__ __launch_bounds__(256) void kFinish(const FrameConst *__restrict__ fcp, BatchDesc b, PathBuffers pb,
                                                const int32_t *done, Counters *cnt, Queue qn, int qsel) {
-    const uint32_t n = cnt->done[qsel ^ 1];
+    const uint32_t n = cnt->done[qsel ^ 1].v;
     finishClears(cnt);
     for (uint32_t base = blockIdx.x * 256; base < n; base += gridDim.x * 256) {
         const uint32_t i = base + threadIdx.x;
@@ -1313,7 +1328,7 @@ __global__ __launch_bounds__(256) void kFinish2(const FrameConst *__restrict__ f
                                                 const FrameConst *__restrict__ fcp2, BatchDesc b2, uint32_t split,
                                                 PathBuffers pb, const int32_t *done, Counters *cnt, Queue qn,
                                                 int qsel) {
-    const uint32_t n = cnt->done[qsel ^ 1];
+    const uint32_t n = cnt->done[qsel ^ 1].v;
     finishClears(cnt);
     for (uint32_t base = blockIdx.x * 256; base < n; base += gridDim.x * 256) {
         const uint32_t i = base + threadIdx.x;
@@ -1327,7 +1342,7 @@ __global__ __launch_bounds__(256) void kFinish2(const FrameConst *__restrict__ f
 // the paths that end leave their slot's live count (one atomic per pass).
 __global__ __launch_bounds__(256) void kFinishM(MultiArgs ma, PathBuffers pb, const int32_t *done, Counters *cnt,
                                                 Queue qn, int qsel) {
-    const uint32_t n = cnt->done[qsel ^ 1];
+    const uint32_t n = cnt->done[qsel ^ 1].v;
     finishClears(cnt);
     for (uint32_t base = blockIdx.x * 256; base < n; base += gridDim.x * 256) {
         const uint32_t i = base + threadIdx.x;
@@ -1338,7 +1353,7 @@ __global__ __launch_bounds__(256) void kFinishM(MultiArgs ma, PathBuffers pb, co
             const bool ended = finishLane(sd.fc, sd.b, pb, done, cnt, qn, qsel, i, true);
             const uint64_t m = __ballot(ended); // the lanes of slot k only
             if (m && (int)__lane_id() == __ffsll((unsigned long long)m) - 1)
-                atomicSub(&ma.slotAlive[k], (uint32_t)__popcll(m));
+                atomicSub(&ma.slotAlive[k].v, (uint32_t)__popcll(m));
         });
     }
 }
@@ -1371,11 +1386,11 @@ __global__ __launch_bounds__(256) void kAccumulate(BatchDesc b, PathBuffers pb, 
 
 __global__ void kResetCounters(Counters *cnt, int which) {
     if (threadIdx.x == 0) {
-        cnt->extend[which] = 0;
-        cnt->shadow = 0;
-        cnt->probe = 0;
-        cnt->done[0] = cnt->done[1] = 0;
-        cnt->fetch[0] = cnt->fetch[1] = cnt->fetch[2] = 0;
+        cnt->extend[which].v = 0;
+        cnt->shadow.v = 0;
+        cnt->probe.v = 0;
+        cnt->done[0].v = cnt->done[1].v = 0;
+        cnt->fetch.v = 0;
     }
 }
 
@@ -1498,7 +1513,7 @@ void launchQueryP(hipStream_t s, const DevScene &S, const rtx_ray *rays, uint32_
     if (closest) hipLaunchKernelGGL(kQueryP<false>, dim3(blocks), dim3(kTraceBlock), 0, s, S, rays, n, out, fetch);
     else hipLaunchKernelGGL(kQueryP<true>, dim3(blocks), dim3(kTraceBlock), 0, s, S, rays, n, out, fetch);
 }
-void launchInstallSlot(hipStream_t s, const SlotDesc &sd, SlotDesc *slots, uint32_t slot, uint32_t *alive) {
+void launchInstallSlot(hipStream_t s, const SlotDesc &sd, SlotDesc *slots, uint32_t slot, CounterWord *alive) {
     hipLaunchKernelGGL(kInstallSlot, dim3(1), dim3(256), 0, s, sd, slots, slot, alive);
 }
 void launchGenerateM(hipStream_t s, const SlotDesc *slots, uint32_t slot, uint32_t numPaths, PathBuffers pb, Queue q0,

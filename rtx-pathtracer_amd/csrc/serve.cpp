@@ -132,7 +132,7 @@ struct rtx_server {
     int32_t *done = nullptr;
     Counters *cnt = nullptr;
     SlotDesc *slotTable = nullptr;
-    uint32_t *slotAlive = nullptr;
+    CounterWord *slotAlive = nullptr;
     uint32_t *ring = nullptr;  // pinned: kPollSlots x (4 + slots) words
     uint32_t ringStride = 0;
     hipEvent_t ringEv[kPollSlots] = {};
@@ -597,7 +597,7 @@ int rtx_server_create(rtx_ctx *ctx, const rtx_server_config *c, rtx_server **out
         return fail(e, "hipHostMalloc (ring)");
     for (hipEvent_t &ev : sv->ringEv)
         if ((e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) return fail(e, "hipEventCreate");
-    launchFillU32(sv->stream, sv->slotAlive, cfg.slots, 0u);
+    launchFillU32(sv->stream, &sv->slotAlive[0].v, cfg.slots * (uint32_t)(sizeof(CounterWord) / 4), 0u);
     if ((e = hipStreamSynchronize(sv->stream)) != hipSuccess) return fail(e, "hipStreamSynchronize");
     rtx_server *raw = sv.release();
     raw->thread = std::thread([raw] { Loop(raw).run(); });
