@@ -1136,6 +1136,7 @@ int rtx_render(rtx_ctx *ctx, const rtx_scene *scene, const rtx_frame_params *p, 
     static const bool logBounces = std::getenv("RTX_LOG_BOUNCES") != nullptr;
     auto bounces = [&](const FrameConst *fcd, BatchDesc b, int iters, bool multi,
                        const PathClass2 *second = nullptr) -> int {
+        const uint32_t features = shadeFeatures(fcd == ctx->fcIC ? fcIC : fc);
         int qsel = 0;
         const int cap = multi ? (int)(samplesPerFrame + kMaxSplits + 1) * (iters + 1) : iters + 1;
         for (int it = 0;; ++it) {
@@ -1167,7 +1168,7 @@ int rtx_render(rtx_ctx *ctx, const rtx_scene *scene, const rtx_frame_params *p, 
             });
             timed(kClsShade, [&] {
                 launchShade(s, S, icv, ctx->guide, fcd, b, ctx->pb, ctx->q[qsel], ctx->q[qsel ^ 1], ctx->qs, ctx->qp,
-                            ctx->done, ctx->cnt, qsel, shadeBlocks, second);
+                            ctx->done, ctx->cnt, qsel, shadeBlocks, features, second);
             });
             qsel ^= 1;
         }

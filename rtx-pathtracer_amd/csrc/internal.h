@@ -371,9 +371,22 @@ struct PathClass2 {
     BatchDesc b;
     uint32_t split;
 };
+// What a frame's shading needs beyond the plain method (launchShade's
+// features); the shading kernel is built for the combinations frames use.
+constexpr uint32_t kShadeIC = 1;        // cache lookups
+constexpr uint32_t kShadeGuide = 2;     // guided directions
+constexpr uint32_t kShadeNrc = 4;       // the learned cache
+constexpr uint32_t kShadeRecord = 8;    // guiding sample records
+constexpr uint32_t kShadeSegments = 16; // frames of several samples, splitting, ADRRS
+constexpr uint32_t kShadeAll = 31;
+inline uint32_t shadeFeatures(const FrameConst &fc) {
+    return (fc.useIC || fc.useADRRS ? kShadeIC : 0u) | (fc.pc.useGuiding ? kShadeGuide : 0u) |
+           (fc.nrc ? kShadeNrc : 0u) | (fc.record ? kShadeRecord : 0u) |
+           (fc.segments || fc.useADRRS || fc.splitOnFirst ? kShadeSegments : 0u);
+}
 void launchShade(hipStream_t s, const DevScene &S, const DevIC &ic, const DevGuiding &g, const FrameConst *fc,
                  BatchDesc b, PathBuffers pb, Queue qin, Queue qout, Queue qs, Queue qp, int32_t *done, Counters *cnt,
-                 int qsel, int blocks, const PathClass2 *second = nullptr);
+                 int qsel, int blocks, uint32_t features, const PathClass2 *second = nullptr);
 // Which jobs of the frame's list a sub-path launch or a reduction covers:
 // [firstJob, firstJob + count) as the host says, or from device memory (the
 // plan's counts, ic.frame[3] updates and ic.frame[4] jobs in all), so that no

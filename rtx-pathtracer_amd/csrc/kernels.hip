@@ -702,14 +702,22 @@ RTX_DI void pushSplit(const PathBuffers &pb, uint32_t pid, int4 &task, const Hit
 }
 
 // ----------------------------------------------------------------- shade
-// Register budget: two waves per SIMD (at most 256 VGPRs and AGPRs
-// together).  Without the bound the compiler reaches 254 VGPRs plus 4 AGPRs
-// and the kernel drops to one wave per SIMD, which costs the 1080p cache
-// workload about 16% (2.35 s per image instead of 2.74 s).
+// Register budget: two waves per SIMD (at most 256 VGPRs), three for a cache
+// frame's two classes (at most 168; 44 cache frames' kShade2: 139 ms with two,
+// 134 with three, 142 with four, which spills 170 registers).  The plain build
+// at 1080p: 0.61 ms a 4.1 M-path launch with two, 0.63 and 0.64 with three and
+// four.
+//
+// The kernel is built for the features a frame uses (launchShade).  One build
+// with all of them kept their parameters and state live through every path,
+// 290 scalar registers spilled instead of 126 to 158: the 256x256 preview's
+// launches took 45 us on average instead of 39, cache frames' 200 instead of 176.
 // One iteration of the bounce loop, raytrace.rgen:1008-1215, for the paths of
 // the extend queue; an entry marked kSplitVertex resumes a queued split
 // instead (raytrace.rgen:1684-1703: NEE at its vertex, a new direction, then
 // the resumed path at the split's depth).
+// F: the features the build contains (kShade*, internal.h).
+template <uint32_t F>
 RTX_DI void shadeLane(const DevScene &S, const DevIC &IC, const DevGuiding &G, const FrameConst &fc,
                       const BatchDesc &b, const PathBuffers &pb, const Queue &qin, const Queue &qout, const Queue &qs,
                       const Queue &qp, int32_t *done, Counters *cnt, int qsel, uint32_t i, bool active) {
@@ -720,11 +728,13 @@ RTX_DI void shadeLane(const DevScene &S, const DevIC &IC, const DevGuiding &G, c
     const bool mis = fc.pc.enableMIS != 0;
     const bool power = fc.pc.usePowerHeuristic != 0;
     const int maxDepth = fc.maxDepth, maxFollow = fc.maxFollow;
-    const bool useIC = fc.useIC != 0, createIC = fc.createIC != 0;
-    const bool record = fc.record != 0;
+    const bool useIC = (F & kShadeIC) && fc.useIC != 0, createIC = (F & kShadeIC) && fc.createIC != 0;
+    const bool record = (F & kShadeRecord) && fc.record != 0;
     const bool icOnGlossy = fc.pc.useIrradianceCacheOnGlossy != 0;
-    const bool segments = fc.segments != 0;
-    const bool useADRRS = fc.useADRRS != 0, splitOnFirst = fc.splitOnFirst != 0;
+    const bool segments = (F & kShadeSegments) && fc.segments != 0;
+    const bool useADRRS = (F & kShadeSegments) && fc.useADRRS != 0;
+    const bool splitOnFirst = (F & kShadeSegments) && fc.splitOnFirst != 0;
+    const bool nrc = (F & kShadeNrc) && fc.nrc != 0;
     const bool adrrsSplit = fc.pc.adrrsSplit != 0;
     const float adrrsS = fc.pc.adrrsS;
     IcQueryParams icp;
@@ -732,7 +742,7 @@ RTX_DI void shadeLane(const DevScene &S, const DevIC &IC, const DevGuiding &G, c
     icp.gradients = fc.pc.useIrradianceGradients != 0;
     icp.visibility = fc.pc.irradianceCachePerformVisibilityCheck != 0;
     GuidingParams gp;
-    gp.on = fc.pc.useGuiding != 0;
+    gp.on = (F & kShadeGuide) && fc.pc.useGuiding != 0;
     gp.parallax = fc.pc.useParallaxCompensation != 0;
     gp.prob = fc.pc.guidingProb;
     uint32_t *nextCount = &cnt->extend[qsel ^ 1].v;
@@ -753,7 +763,7 @@ RTX_DI void shadeLane(const DevScene &S, const DevIC &IC, const DevGuiding &G, c
     float firstT = kTMax;
     if (active) {
         const uint32_t raw = (uint32_t)qin.id[i];
-        splitV = (raw & kSplitVertex) != 0;
+        splitV = (F & kShadeSegments) && (raw & kSplitVertex) != 0;
         pid = raw & ~kSplitVertex;
         float4 hit = qin.hit[i];
         d = v3(qin.dir[i]);
@@ -783,7 +793,7 @@ RTX_DI void shadeLane(const DevScene &S, const DevIC &IC, const DevGuiding &G, c
         }
         if (flags & kFlagPending) {
             V3 nee = pendingSum(pb, pid, numNEE, fc.neeStride, hash, sh0, pr0);
-            if (flags & kFlagPendTask) { // a split vertex's NEE joins main()'s result
+            if ((F & kShadeSegments) && (flags & kFlagPendTask)) { // a split vertex's NEE joins main()'s result
                 float4 tr = pb.taskRes[pid];
                 pb.taskRes[pid] = f4(v3(tr) + nee, tr.w);
             } else if (record) { // recorded NEE terms are kept without the throughput
@@ -859,7 +869,7 @@ RTX_DI void shadeLane(const DevScene &S, const DevIC &IC, const DevGuiding &G, c
                 addNext = false;
                 follow = false;
                 bool nee = useNEE;
-                if (fc.nrc && depth >= (int)fc.nrcDepth && !(flags & kFlagNrcTrain)) {
+                if (nrc && depth >= (int)fc.nrcDepth && !(flags & kFlagNrcTrain)) {
                     const int slot = nrcSlot(fc, b, pid);
                     if (slot < 0) { // the path ends into the learned cache here, without NEE
                         nrcQ = true;
@@ -878,7 +888,7 @@ RTX_DI void shadeLane(const DevScene &S, const DevIC &IC, const DevGuiding &G, c
                         pb.nrcPath[2 * (size_t)pid + 1] = f4(res, __int_as_float(depth));
                         flags |= kFlagNrcTrain;
                     }
-                } else if (fc.nrcSuffix && (flags & kFlagNrcTrain) && !(flags & kFlagNrcTrainEnd)) {
+                } else if (nrc && fc.nrcSuffix && (flags & kFlagNrcTrain) && !(flags & kFlagNrcTrainEnd)) {
                     // self-training: the suffix ends into the cache nrcSuffix vertices past the
                     // training vertex; the cache's prediction there completes the target
                     const int d0 = __float_as_int(pb.nrcPath[2 * (size_t)pid + 1].w);
@@ -1049,7 +1059,7 @@ RTX_DI void shadeLane(const DevScene &S, const DevIC &IC, const DevGuiding &G, c
             qp.aux[pi] = f4(probeBase, pdfMatProbe);
         }
     }
-    if (fc.nrc) { // the learned cache's queries, in the order the waves reach them
+    if (nrc) { // the learned cache's queries, in the order the waves reach them
         const int qn = waveAppend(nrcQ, pb.nrcQueryCount);
         if (nrcQ) {
             float rough;
@@ -1155,6 +1165,7 @@ RTX_DI void shadeLane(const DevScene &S, const DevIC &IC, const DevGuiding &G, c
     if (isDone) done[di] = (int)pid;
 }
 
+template <uint32_t F>
 __global__ __launch_bounds__(kShadeBlock, 2) void kShade(DevScene S, DevIC IC, DevGuiding G,
                                                       const FrameConst *__restrict__ fcp, BatchDesc b, PathBuffers pb,
                                                       Queue qin, Queue qout, Queue qs, Queue qp, int32_t *done,
@@ -1162,14 +1173,15 @@ __global__ __launch_bounds__(kShadeBlock, 2) void kShade(DevScene S, DevIC IC, D
     const uint32_t n = cnt->extend[qsel].v;
     for (uint32_t base = blockIdx.x * kShadeBlock; base < n; base += gridDim.x * kShadeBlock) {
         const uint32_t i = base + threadIdx.x;
-        shadeLane(S, IC, G, *fcp, b, pb, qin, qout, qs, qp, done, cnt, qsel, i, i < n);
+        shadeLane<F>(S, IC, G, *fcp, b, pb, qin, qout, qs, qp, done, cnt, qsel, i, i < n);
     }
 }
 
 // Two classes of paths in one wavefront: ids below `split` are the class of
 // (fc, b), the others of (fc2, b2) (a frame's camera paths and the cache's
 // update sub-paths).  A wave takes one pass per class among its lanes.
-__global__ __launch_bounds__(kShadeBlock, 2) void kShade2(DevScene S, DevIC IC, DevGuiding G,
+template <uint32_t F>
+__global__ __launch_bounds__(kShadeBlock, 3) void kShade2(DevScene S, DevIC IC, DevGuiding G,
                                                        const FrameConst *__restrict__ fcp, BatchDesc b,
                                                        const FrameConst *__restrict__ fcp2, BatchDesc b2,
                                                        uint32_t split, PathBuffers pb, Queue qin, Queue qout,
@@ -1180,7 +1192,7 @@ __global__ __launch_bounds__(kShadeBlock, 2) void kShade2(DevScene S, DevIC IC, 
         const bool active = i < n;
         const uint32_t cls = active && ((uint32_t)qin.id[i] & ~kSplitVertex) >= split ? 1u : 0u;
         forEachKey(active, cls, [&](uint32_t k) {
-            shadeLane(S, IC, G, k ? *fcp2 : *fcp, k ? b2 : b, pb, qin, qout, qs, qp, done, cnt, qsel, i, true);
+            shadeLane<F>(S, IC, G, k ? *fcp2 : *fcp, k ? b2 : b, pb, qin, qout, qs, qp, done, cnt, qsel, i, true);
         });
     }
 }
@@ -1199,7 +1211,7 @@ __global__ __launch_bounds__(kShadeBlock, 2) void kShadeM(MultiArgs ma, PathBuff
         const uint32_t slot = active ? ((uint32_t)qin.id[i] & ~kSplitVertex) >> ma.slotShift : 0u;
         forEachKey(active, slot, [&](uint32_t k) {
             const SlotDesc &sd = ma.slots[k];
-            shadeLane(sd.S, sd.ic, sd.g, sd.fc, sd.b, pb, qin, qout, qs, qp, done, cnt, qsel, i, true);
+            shadeLane<kShadeIC | kShadeGuide>(sd.S, sd.ic, sd.g, sd.fc, sd.b, pb, qin, qout, qs, qp, done, cnt, qsel, i, true);
         });
     }
 }
@@ -1482,13 +1494,21 @@ void launchProbeResolve(hipStream_t s, const DevScene &S, const FrameConst *fc, 
 }
 void launchShade(hipStream_t s, const DevScene &S, const DevIC &ic, const DevGuiding &g, const FrameConst *fc,
                  BatchDesc b, PathBuffers pb, Queue qin, Queue qout, Queue qs, Queue qp, int32_t *done, Counters *cnt,
-                 int qsel, int blocks, const PathClass2 *second) {
-    if (second)
-        hipLaunchKernelGGL(kShade2, dim3(blocks), dim3(kShadeBlock), 0, s, S, ic, g, fc, b, second->fc, second->b,
-                           second->split, pb, qin, qout, qs, qp, done, cnt, qsel);
-    else
-        hipLaunchKernelGGL(kShade, dim3(blocks), dim3(kShadeBlock), 0, s, S, ic, g, fc, b, pb, qin, qout, qs, qp, done,
-                           cnt, qsel);
+                 int qsel, int blocks, uint32_t features, const PathClass2 *second) {
+    const dim3 grid(blocks), t(kShadeBlock);
+    if (second) {
+        // a frame with its cache upkeep: no records, segments or learned cache
+        auto k = features & kShadeGuide ? kShade2<kShadeIC | kShadeGuide> : kShade2<kShadeIC>;
+        hipLaunchKernelGGL(k, grid, t, 0, s, S, ic, g, fc, b, second->fc, second->b, second->split, pb, qin, qout, qs,
+                           qp, done, cnt, qsel);
+        return;
+    }
+    auto k = kShade<kShadeAll>;
+    if (features == 0u) k = kShade<0u>;
+    else if ((features & ~kShadeIC) == 0u) k = kShade<kShadeIC>;
+    else if ((features & ~kShadeGuide) == 0u) k = kShade<kShadeGuide>;
+    else if ((features & ~kShadeNrc) == 0u) k = kShade<kShadeNrc>;
+    hipLaunchKernelGGL(k, grid, t, 0, s, S, ic, g, fc, b, pb, qin, qout, qs, qp, done, cnt, qsel);
 }
 void launchFinish(hipStream_t s, const FrameConst *fc, BatchDesc b, PathBuffers pb, const int32_t *done,
                   Counters *cnt, Queue qnext, int qsel, int blocks, const PathClass2 *second) {
