@@ -21,6 +21,8 @@
 //   kToVmm      VMM_Theta for rendering (syncPMMsToVMM_Thetas, 117-139)
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "dev_math.h"
 #include "dev_sort.h"
 #include "internal.h"
@@ -82,13 +84,19 @@ __global__ __launch_bounds__(kSortBlock) void kCompactScatter(const rtx_directio
     }
 }
 
-__global__ __launch_bounds__(256) void kSegmentCount(const uint32_t *keys, const uint32_t *count, uint32_t *regionCount) {
+// regionStart[r], r = 0..numRegions: the first of the sorted keys that is r or
+// more.  Each sample whose key differs from the one before it writes the
+// starts in between, so every start is written once and none is contended
+// (counting a region's samples with atomics took 3.0 ms for the spot room's
+// 640x360 frames, whose samples fall into few regions at a time; this 9 us).
+__global__ __launch_bounds__(256) void kSegments(const uint32_t *keys, const uint32_t *count, uint32_t numRegions,
+                                                 uint32_t *regionStart) {
     const uint32_t n = *count;
-    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) atomicAdd(&regionCount[keys[i]], 1u);
-}
-
-__global__ __launch_bounds__(256) void kZero(uint32_t *a, uint32_t n) {
-    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) a[i] = 0;
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i <= n; i += gridDim.x * 256) {
+        const uint32_t hi = i < n ? keys[i] : numRegions; // the last start at or below sample i
+        uint32_t r = i > 0 ? keys[i - 1] + 1u : 0u;
+        for (; r <= hi; ++r) regionStart[r] = i;
+    }
 }
 
 // --------------------------------------------------------------- preFit
@@ -155,26 +163,46 @@ RTX_DI double waveSumD(double v) {
     return v;
 }
 
+// The loops over a mixture's lobes below run to a compile-time KM (8, 16 or
+// 32: the least that holds K), unrolled up to 16, with the lobes past K
+// branched over, so that the per-lobe sums of a thread stay in registers;
+// indexed by a loop to K they live in scratch memory, and the sample loops
+// waited for them (spot room, 640x360, 256 regions: kRegionEM 1.27 ms,
+// kSplitMerge 3.1 ms; now 0.42 and 1.08 ms).  32 lobes' sums do not fit the
+// registers and stay in scratch.
+template <int KM> constexpr int kUnroll = KM <= 16 ? KM : 1;
+template <class F> RTX_DI void withLobes(int K, F &&f) {
+    if (K <= 8) f(std::integral_constant<int, 8>{});
+    else if (K <= 16) f(std::integral_constant<int, 16>{});
+    else f(std::integral_constant<int, kK>{});
+}
+
 // E-step over the region's samples with the model in LDS; leaves the
 // block totals in E.tot.
-RTX_DI void eStep(EmShared &E, int K, const float4 *smp, uint32_t n) {
-    float W[kK], RW[kK][3];
-    for (int k = 0; k < kK; ++k) W[k] = RW[k][0] = RW[k][1] = RW[k][2] = 0.0f;
+template <int KM> RTX_DI void eStepLobes(EmShared &E, int K, const float4 *smp, uint32_t n) {
+    constexpr int UN = kUnroll<KM>;
+    float W[KM], RW[KM][3];
+#pragma unroll UN
+    for (int k = 0; k < KM; ++k) W[k] = RW[k][0] = RW[k][1] = RW[k][2] = 0.0f;
     float sumW = 0.0f;
     double ll = 0.0;
     for (uint32_t j = threadIdx.x; j < n; j += kEmBlock) {
         const float4 a4 = smp[2 * j];
         const V3 d = v3(a4);
-        float a[kK];
+        float a[KM];
         float total = 0.0f;
-        for (int k = 0; k < K; ++k) {
+#pragma unroll UN
+        for (int k = 0; k < KM; ++k) {
+            if (k >= K) continue;
             const float c = E.mu[k][0] * d.x + E.mu[k][1] * d.y + E.mu[k][2] * d.z;
             a[k] = E.w[k] * (E.norm[k] * fastexpf(E.kappa[k] * fminf(c - 1.0f, 0.0f)));
             total += a[k];
         }
         if (!(total > 1e-8f)) continue; // SoftAssignmentWeights::valid
         const float inv = 1.0f / total;
-        for (int k = 0; k < K; ++k) {
+#pragma unroll UN
+        for (int k = 0; k < KM; ++k) {
+            if (k >= K) continue;
             const float aw = a[k] * inv * a4.w;
             RW[k][0] += d.x * aw;
             RW[k][1] += d.y * aw;
@@ -185,7 +213,9 @@ RTX_DI void eStep(EmShared &E, int K, const float4 *smp, uint32_t n) {
         ll += (double)a4.w * (double)logf(total);
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int k = 0; k < K; ++k) {
+#pragma unroll UN
+    for (int k = 0; k < KM; ++k) {
+        if (k >= K) continue;
         double v0 = waveSumD(W[k]), v1 = waveSumD(RW[k][0]), v2 = waveSumD(RW[k][1]), v3_ = waveSumD(RW[k][2]);
         if (lane == 0) {
             E.stat[wave][4 * k] = v0;
@@ -206,6 +236,10 @@ RTX_DI void eStep(EmShared &E, int K, const float4 *smp, uint32_t n) {
         E.tot[t] = acc;
     }
     __syncthreads();
+}
+
+RTX_DI void eStep(EmShared &E, int K, const float4 *smp, uint32_t n) {
+    withLobes(K, [&](auto km) { eStepLobes<decltype(km)::value>(E, K, smp, n); });
 }
 
 RTX_DI float applyWeightPrior(const EmProps &P, float w, int K) {
@@ -600,7 +634,7 @@ struct SmShared {
     int pairA[kK * (kK - 1) / 2], pairB[kK * (kK - 1) / 2];
     int mask[kK];
     float oldActive, sumWeight, norm;
-    int numSplits, stop;
+    int numSplits, stop, nValid;
 };
 
 RTX_DI void loadModel(EmShared &E, const GuideRegion &R) {
@@ -613,6 +647,58 @@ RTX_DI void loadModel(EmShared &E, const GuideRegion &R) {
         for (int c = 0; c < 3; ++c) E.mu[k][c] = R.mu[k][c];
     }
     __syncthreads();
+}
+
+// The sample sums of chiCovUpdate, to S.part.
+template <int KM> RTX_DI void chiCovSums(SmShared &S, int K, const float4 *smp, uint32_t n, bool useMask) {
+    constexpr int UN = kUnroll<KM>;
+    EmShared &E = S.E;
+    float chiB[KM], bw[KM], bv[KM][3];
+#pragma unroll UN
+    for (int k = 0; k < KM; ++k) chiB[k] = bw[k] = bv[k][0] = bv[k][1] = bv[k][2] = 0.0f;
+    for (uint32_t j = threadIdx.x; j < n; j += kEmBlock) {
+        const float4 a4 = smp[2 * j];
+        const float pdf = smp[2 * j + 1].y;
+        const V3 d = v3(a4);
+        float p[KM], mix = 0.0f;
+#pragma unroll UN
+        for (int k = 0; k < KM; ++k) {
+            if (k >= K) continue;
+            const float c = E.mu[k][0] * d.x + E.mu[k][1] * d.y + E.mu[k][2] * d.z;
+            p[k] = E.norm[k] * fastexpf(E.kappa[k] * fminf(c - 1.0f, 0.0f));
+            mix += E.w[k] * p[k];
+        }
+        if (!(mix > 1e-8f)) continue; // PMM_EPSILON
+        const float f = a4.w * a4.w * pdf / (mix * mix);
+        const float inv = 1.0f / mix;
+#pragma unroll UN
+        for (int k = 0; k < KM; ++k) {
+            if (k >= K) continue;
+            if (useMask && !S.mask[k]) continue;
+            chiB[k] += p[k] * f;
+            const float ws = a4.w * (E.w[k] * p[k] * inv);
+            bw[k] += ws;
+            const float lx = S.fs[k][0] * d.x + S.fs[k][1] * d.y + S.fs[k][2] * d.z;
+            const float ly = S.ft[k][0] * d.x + S.ft[k][1] * d.y + S.ft[k][2] * d.z;
+            bv[k][0] += lx * lx * ws;
+            bv[k][1] += ly * ly * ws;
+            bv[k][2] += lx * ly * ws;
+        }
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll UN
+    for (int k = 0; k < KM; ++k) {
+        if (k >= K) continue;
+        const double v0 = waveSumD(chiB[k]), v1 = waveSumD(bw[k]), v2 = waveSumD(bv[k][0]), v3_ = waveSumD(bv[k][1]),
+                     v4 = waveSumD(bv[k][2]);
+        if (lane == 0) {
+            S.part[wave][5 * k] = v0;
+            S.part[wave][5 * k + 1] = v1;
+            S.part[wave][5 * k + 2] = v2;
+            S.part[wave][5 * k + 3] = v3_;
+            S.part[wave][5 * k + 4] = v4;
+        }
+    }
 }
 
 // IncrementalPearsonChiSquared::updateDivergence(Masked) (54-148) and
@@ -636,45 +722,7 @@ RTX_DI void chiCovUpdate(SmShared &S, GuideRegion &R, const float4 *smp, uint32_
         S.fs[k][2] = t[0] * nn[1] - t[1] * nn[0];
     }
     __syncthreads();
-    float chiB[kK], bw[kK], bv[kK][3];
-    for (int k = 0; k < kK; ++k) chiB[k] = bw[k] = bv[k][0] = bv[k][1] = bv[k][2] = 0.0f;
-    for (uint32_t j = threadIdx.x; j < n; j += kEmBlock) {
-        const float4 a4 = smp[2 * j];
-        const float pdf = smp[2 * j + 1].y;
-        const V3 d = v3(a4);
-        float p[kK], mix = 0.0f;
-        for (int k = 0; k < K; ++k) {
-            const float c = E.mu[k][0] * d.x + E.mu[k][1] * d.y + E.mu[k][2] * d.z;
-            p[k] = E.norm[k] * fastexpf(E.kappa[k] * fminf(c - 1.0f, 0.0f));
-            mix += E.w[k] * p[k];
-        }
-        if (!(mix > 1e-8f)) continue; // PMM_EPSILON
-        const float f = a4.w * a4.w * pdf / (mix * mix);
-        const float inv = 1.0f / mix;
-        for (int k = 0; k < K; ++k) {
-            if (useMask && !S.mask[k]) continue;
-            chiB[k] += p[k] * f;
-            const float ws = a4.w * (E.w[k] * p[k] * inv);
-            bw[k] += ws;
-            const float lx = S.fs[k][0] * d.x + S.fs[k][1] * d.y + S.fs[k][2] * d.z;
-            const float ly = S.ft[k][0] * d.x + S.ft[k][1] * d.y + S.ft[k][2] * d.z;
-            bv[k][0] += lx * lx * ws;
-            bv[k][1] += ly * ly * ws;
-            bv[k][2] += lx * ly * ws;
-        }
-    }
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int k = 0; k < K; ++k) {
-        const double v0 = waveSumD(chiB[k]), v1 = waveSumD(bw[k]), v2 = waveSumD(bv[k][0]), v3_ = waveSumD(bv[k][1]),
-                     v4 = waveSumD(bv[k][2]);
-        if (lane == 0) {
-            S.part[wave][5 * k] = v0;
-            S.part[wave][5 * k + 1] = v1;
-            S.part[wave][5 * k + 2] = v2;
-            S.part[wave][5 * k + 3] = v3_;
-            S.part[wave][5 * k + 4] = v4;
-        }
-    }
+    withLobes(K, [&](auto km) { chiCovSums<decltype(km)::value>(S, K, smp, n, useMask); });
     __syncthreads();
     if (threadIdx.x < (unsigned)K && (!useMask || S.mask[threadIdx.x])) {
         const int k = threadIdx.x;
@@ -764,7 +812,12 @@ __global__ __launch_bounds__(kEmBlock) void kSplitMerge(GuideFitBuffers g, EmPro
     const uint32_t r = blockIdx.x;
     const uint32_t s0 = g.regionStart[r], n = g.regionStart[r + 1] - s0;
     if (n == 0) return;
-    GuideRegion &R = g.regions[r];
+    // the region is edited in LDS: lane 0's edits are chains of dependent reads
+    __shared__ GuideRegion R;
+    static_assert(sizeof(GuideRegion) % 4 == 0, "copied as words");
+    for (uint32_t t = threadIdx.x; t < sizeof(GuideRegion) / 4; t += kEmBlock)
+        reinterpret_cast<uint32_t *>(&R)[t] = reinterpret_cast<const uint32_t *>(g.regions + r)[t];
+    __syncthreads();
     const float4 *smp = g.samples + 2 * (size_t)s0;
     // ---- mergeAll (635-709)
     const bool doMerge = R.samplesSinceLastMerge + n > SP.minSamplesForMerging;
@@ -800,18 +853,33 @@ __global__ __launch_bounds__(kEmBlock) void kSplitMerge(GuideFitBuffers g, EmPro
                     S.pairA[last] = ta, S.pairB[last] = tb;
                     ++first;
                 }
-                const int nValid = first;
-                // stable insertion sort by metric, ascending
-                for (int q = 1; q < nValid; ++q) {
-                    const float m = S.metric[q];
-                    const int a = S.pairA[q], b = S.pairB[q];
-                    int p = q - 1;
-                    while (p >= 0 && S.metric[p] > m) {
-                        S.metric[p + 1] = S.metric[p], S.pairA[p + 1] = S.pairA[p], S.pairB[p + 1] = S.pairB[p];
-                        --p;
-                    }
-                    S.metric[p + 1] = m, S.pairA[p + 1] = a, S.pairB[p + 1] = b;
+                S.nValid = first;
+            }
+            __syncthreads();
+            // stable sort by metric, ascending: each pair's place is the number
+            // of pairs before it (lane 0's insertion sort waited for LDS at
+            // every step)
+            const int nValid = S.nValid;
+            static_assert(kK * (kK - 1) / 2 <= 2 * kEmBlock, "two pairs a thread");
+            float sm[2];
+            int sa[2], sb[2], place[2];
+            for (int h = 0; h < 2; ++h) {
+                const int q = threadIdx.x + h * kEmBlock;
+                if (q >= nValid) continue;
+                sm[h] = S.metric[q], sa[h] = S.pairA[q], sb[h] = S.pairB[q];
+                int before = 0;
+                for (int t = 0; t < nValid; ++t) {
+                    const float m = S.metric[t];
+                    before += m < sm[h] || (m == sm[h] && t < q) ? 1 : 0;
                 }
+                place[h] = before;
+            }
+            __syncthreads();
+            for (int h = 0; h < 2; ++h)
+                if (threadIdx.x + h * kEmBlock < (unsigned)nValid)
+                    S.metric[place[h]] = sm[h], S.pairA[place[h]] = sa[h], S.pairB[place[h]] = sb[h];
+            __syncthreads();
+            if (threadIdx.x == 0) {
                 uint32_t used = 0;
                 int ma[kK], mb[kK], nm = 0;
                 for (int q = 0; q < nValid; ++q) {
@@ -913,6 +981,9 @@ __global__ __launch_bounds__(kEmBlock) void kSplitMerge(GuideFitBuffers g, EmPro
     }
     __syncthreads();
     if (threadIdx.x == 0) pmmApplyPrior(R, P.vPrior);
+    __syncthreads();
+    for (uint32_t t = threadIdx.x; t < sizeof(GuideRegion) / 4; t += kEmBlock)
+        reinterpret_cast<uint32_t *>(g.regions + r)[t] = reinterpret_cast<const uint32_t *>(&R)[t];
 }
 
 // incrementaldistance.h:58-104
@@ -1085,9 +1156,7 @@ void launchGuideUpdate(hipStream_t s, GuideFitBuffers g, const rtx_directional_d
         std::swap(g.valsA, g.valsB);
     }
     // region segments
-    hipLaunchKernelGGL(kZero, dim3(blocksOf(g.numRegions + 1, 256)), dim3(256), 0, s, g.regionStart, g.numRegions + 1);
-    hipLaunchKernelGGL(kSegmentCount, dim3(1024), dim3(256), 0, s, g.keysA, g.counters, g.regionStart);
-    hipLaunchKernelGGL(kScanInPlace<0>, dim3(1), dim3(1024), 0, s, g.regionStart, g.numRegions + 1, (uint32_t *)nullptr);
+    hipLaunchKernelGGL(kSegments, dim3(1024), dim3(256), 0, s, g.keysA, g.counters, g.numRegions, g.regionStart);
     // preFit, EM, distances
     hipLaunchKernelGGL(kPrefit, dim3(blocksOf(g.numRegions, 64)), dim3(64), 0, s, g, parallax, firstFit);
     hipLaunchKernelGGL(kGather, dim3(1024), dim3(256), 0, s, g, dd, parallax);
