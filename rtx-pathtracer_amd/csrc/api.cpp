@@ -625,28 +625,39 @@ int rtx_scene_create(rtx_ctx *ctx, const rtx_scene_desc *d, rtx_scene **out) try
     DevScene &S = sc->view;
     hipError_t e = hipSuccess;
     float4 *nodes = nullptr, *trisD = nullptr;
-    int4 *prD = nullptr;
+    float4 *prD = nullptr;
     rtx_vertex *vD = nullptr;
     uint32_t *iD = nullptr, *vbD = nullptr, *ibD = nullptr;
     rtx_instance *instD = nullptr;
     rtx_material *matD = nullptr;
     rtx_light *lightD = nullptr;
-    int32_t *liD = nullptr;
+    uint32_t *liD = nullptr;
     rtx_face_sample *ftD = nullptr;
     rtx_sphere *spD = nullptr;
     if (e == hipSuccess) e = upload(&nodes, reinterpret_cast<const float4 *>(bvh.nodes.data()), bvh.nodes.size() * kWideNodeSlots);
     if (e == hipSuccess) e = upload(&trisD, tris.data(), tris.size());
     float4 *lightTrisD = nullptr;
     if (e == hipSuccess && lightTrisOk && !lightTris.empty()) e = upload(&lightTrisD, lightTris.data(), lightTris.size());
-    // per world triangle: its instance and the global indices of its vertices
-    std::vector<int4> triRef((size_t)numTris);
+    // per world triangle: its vertices, material and instance (DevScene::triShade)
+    std::vector<float4> triShade((size_t)numTris * kTriShadeSlots, make_float4(0.0f, 0.0f, 0.0f, 0.0f));
+    auto intBits = [](int32_t i) {
+        float f;
+        std::memcpy(&f, &i, 4);
+        return f;
+    };
     for (size_t p = 0; p < (size_t)numTris; ++p) {
-        const int inst = primRef[p].x;
-        const int model = d->instances[inst].modelIndex;
-        const uint32_t *ix = d->models[model].indices + 3 * (size_t)primRef[p].y;
-        triRef[p] = make_int4(inst, (int)(vbase[model] + ix[0]), (int)(vbase[model] + ix[1]), (int)(vbase[model] + ix[2]));
+        const rtx_instance &in = d->instances[primRef[p].x];
+        const rtx_model_desc &md = d->models[in.modelIndex];
+        const uint32_t *ix = md.indices + 3 * (size_t)primRef[p].y;
+        float4 *o = &triShade[kTriShadeSlots * p];
+        for (int k = 0; k < 3; ++k) {
+            const rtx_vertex &v = md.vertices[ix[k]];
+            o[2 * k] = make_float4(v.pos[0], v.pos[1], v.pos[2], v.normal[0]);
+            o[2 * k + 1] = make_float4(v.normal[1], v.normal[2], v.texCoord[0], v.texCoord[1]);
+        }
+        o[6] = make_float4(intBits(md.vertices[ix[0]].materialIndex), intBits(primRef[p].x), intBits(in.iLight), 0.0f);
     }
-    if (e == hipSuccess) e = upload(&prD, triRef.data(), triRef.size());
+    if (e == hipSuccess) e = upload(&prD, triShade.data(), triShade.size());
     if (e == hipSuccess) e = upload(&vD, verts.data(), verts.size());
     if (e == hipSuccess) e = upload(&iD, idx.data(), idx.size());
     if (e == hipSuccess) e = upload(&vbD, vbase.data(), vbase.size());
@@ -654,7 +665,26 @@ int rtx_scene_create(rtx_ctx *ctx, const rtx_scene_desc *d, rtx_scene **out) try
     if (e == hipSuccess) e = upload(&instD, d->instances, d->instanceCount);
     if (e == hipSuccess) e = upload(&matD, d->materials, d->materialCount);
     if (e == hipSuccess) e = upload(&lightD, d->lights, d->lightCount);
-    if (e == hipSuccess) e = upload(&liD, d->randomLightIndex, d->lightCount ? RTX_SIZE_LIGHT_RANDOM : 0);
+    // the random light table with each light's type, so that its branch does
+    // not wait for the light
+    std::vector<uint32_t> lightTable(d->lightCount ? RTX_SIZE_LIGHT_RANDOM : 0);
+    for (size_t i = 0; i < lightTable.size(); ++i) {
+        const uint32_t l = (uint32_t)d->randomLightIndex[i];
+        lightTable[i] = l | (uint32_t)d->lights[l].type << kLightTypeShift;
+    }
+    if (e == hipSuccess) e = upload(&liD, lightTable.data(), lightTable.size());
+    std::vector<float4> lightSpheres;
+    std::vector<int32_t> lightSphereId;
+    for (uint32_t k = 0; k < d->sphereCount; ++k) {
+        const rtx_sphere &sp = d->spheres[k];
+        if (d->materials[sp.materialIndex].type != RTX_MAT_LIGHT) continue;
+        lightSpheres.push_back(make_float4(sp.center[0], sp.center[1], sp.center[2], sp.radius));
+        lightSphereId.push_back((int32_t)((uint32_t)numTris + k));
+    }
+    float4 *lsD = nullptr;
+    int32_t *lsIdD = nullptr;
+    if (e == hipSuccess) e = upload(&lsD, lightSpheres.data(), lightSpheres.size());
+    if (e == hipSuccess) e = upload(&lsIdD, lightSphereId.data(), lightSphereId.size());
     if (e == hipSuccess)
         e = upload(&ftD, d->randomTriIndex, d->randomTriIndex ? (size_t)d->randomTriRows * RTX_SIZE_TRI_RANDOM : 0);
     if (e == hipSuccess) e = upload(&spD, d->spheres, d->sphereCount);
@@ -719,7 +749,7 @@ int rtx_scene_create(rtx_ctx *ctx, const rtx_scene_desc *d, rtx_scene **out) try
     }
     S.nodes = nodes;
     S.tris = trisD;
-    S.triRef = prD;
+    S.triShade = prD;
     S.vertices = vD;
     S.indices = iD;
     S.vertexBase = vbD;
@@ -733,6 +763,9 @@ int rtx_scene_create(rtx_ctx *ctx, const rtx_scene_desc *d, rtx_scene **out) try
     S.lightInst = linstD;
     S.lightTris = lightTrisOk ? lightTrisD : nullptr;
     S.numLightTris = lightTrisOk ? (uint32_t)(lightTris.size() / 3) : 0u;
+    S.lightSpheres = lsD;
+    S.lightSphereId = lsIdD;
+    S.numLightSpheres = (uint32_t)lightSpheres.size();
     S.lightFirstOk = lightTrisOk ? 1u : 0u;
     S.spheres = spD;
     S.numTris = (uint32_t)numTris;
@@ -753,7 +786,7 @@ int rtx_scene_create(rtx_ctx *ctx, const rtx_scene_desc *d, rtx_scene **out) try
     sc->info.nodes = (uint32_t)bvh.nodes.size();
     sc->info.maxDepth = bvh.maxDepth;
     sc->info.deviceBytes = bvh.nodes.size() * sizeof(Bvh8Node) + tris.size() * sizeof(float4) +
-                           primRef.size() * sizeof(int4) + verts.size() * sizeof(rtx_vertex) +
+                           triShade.size() * sizeof(float4) + verts.size() * sizeof(rtx_vertex) +
                            idx.size() * 4 + (size_t)d->materialCount * sizeof(rtx_material);
     sc->info.buildMs = buildMs;
     for (int a = 0; a < 3; ++a) {

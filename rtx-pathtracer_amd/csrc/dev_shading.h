@@ -343,6 +343,7 @@ struct HitInfo {
     float u, v;
     int matIndex;
     int instanceIndex;
+    int iLight; // the light the primitive belongs to
     bool frontFace, isSphere;
 };
 
@@ -361,20 +362,24 @@ RTX_DI HitInfo hitInfo(const DevScene &S, int prim, float t, float bu, float bv,
         h.matIndex = s.materialIndex;
         h.isSphere = true;
         h.instanceIndex = si;
+        h.iLight = s.iLight;
     } else {
-        const int4 ref = S.triRef[prim]; // one load instead of the instance -> index -> vertex chain
-        const rtx_instance &in = S.instances[ref.x];
-        const rtx_vertex &v0 = S.vertices[ref.y], &v1 = S.vertices[ref.z], &v2 = S.vertices[ref.w];
+        // one line holds what the hit needs (the instance, index and vertex
+        // arrays: three dependent loads over five lines)
+        const float4 *ts = S.triShade + kTriShadeSlots * (size_t)prim;
+        const float4 a0 = ts[0], c0 = ts[1], a1 = ts[2], c1 = ts[3], a2 = ts[4], c2 = ts[5], ref = ts[6];
+        const rtx_instance &in = S.instances[__float_as_int(ref.y)];
         float b0 = 1.0f - bu - bv;
-        normal = v3(v0.normal) * b0 + v3(v1.normal) * bu + v3(v2.normal) * bv;
+        normal = v3(a0.w, c0.x, c0.y) * b0 + v3(a1.w, c1.x, c1.y) * bu + v3(a2.w, c2.x, c2.y) * bv;
         normal = normalize(xform(in.normalTransform, normal, 0.0f));
-        V3 wp = v3(v0.pos) * b0 + v3(v1.pos) * bu + v3(v2.pos) * bv;
+        V3 wp = v3(a0) * b0 + v3(a1) * bu + v3(a2) * bv;
         h.worldPos = xform(in.transform, wp, 1.0f);
-        h.u = v0.texCoord[0] * b0 + v1.texCoord[0] * bu + v2.texCoord[0] * bv;
-        h.v = v0.texCoord[1] * b0 + v1.texCoord[1] * bu + v2.texCoord[1] * bv;
-        h.matIndex = v0.materialIndex;
+        h.u = c0.z * b0 + c1.z * bu + c2.z * bv;
+        h.v = c0.w * b0 + c1.w * bu + c2.w * bv;
+        h.matIndex = __float_as_int(ref.x);
+        h.instanceIndex = __float_as_int(ref.y);
+        h.iLight = __float_as_int(ref.z);
         h.isSphere = false;
-        h.instanceIndex = ref.x;
     }
     if (dot(d, normal) < 0.0f) {
         h.frontFace = true;
@@ -390,22 +395,23 @@ RTX_DI HitInfo hitInfo(const DevScene &S, int prim, float t, float bu, float bv,
 RTX_DI float sampleLights(const DevScene &S, Rng &r, V3 origin, V3 normal, V3 &lightDir, V3 &lightColor,
                           float &lightDist) {
     int iRandomLight = r.integer(RTX_SIZE_LIGHT_RANDOM - 1);
-    int iLight = S.lightIndex[iRandomLight];
+    const uint32_t row = S.lightIndex[iRandomLight];
+    const int iLight = (int)(row & kLightRowMask), type = (int)(row >> kLightTypeShift);
     const rtx_light &light = S.lights[iLight];
-    if (light.type == RTX_LIGHT_ENV_MAP) { // raytrace.rgen:406-421: uniform hemisphere, pdf 1 / 2pi
+    if (type == RTX_LIGHT_ENV_MAP) { // raytrace.rgen:406-421: uniform hemisphere, pdf 1 / 2pi
         lightDir = randomInHemisphere(r, normal);
         lightColor = envColor(S, lightDir);
         lightDist = kTMax;
         return light.sampleProb / (2.0f * kPi);
     }
-    if (light.type == RTX_LIGHT_POINT) {
+    if (type == RTX_LIGHT_POINT) {
         V3 toLight = v3(light.pos) - origin;
         lightDist = length(toLight);
         lightDir = toLight / lightDist;
         lightColor = v3(light.color) / (lightDist * lightDist);
         return light.sampleProb;
     }
-    if (light.type == RTX_LIGHT_SPHERE) {
+    if (type == RTX_LIGHT_SPHERE) {
         const rtx_sphere &s = S.spheres[light.instanceIndex];
         lightColor = v3(S.materials[s.materialIndex].lightColor);
         V3 sphereNormal;

@@ -83,13 +83,13 @@ RTX_DI uint32_t satU32(float x) {
 // t), randomUInt) (GLSL's uint(vec2) takes the first component).
 RTX_DI bool alphaAccept(const DevScene &S, int prim, float ox, float t, float bu, float bv, uint32_t randomUInt) {
 #pragma clang fp contract(off)
-    const int4 ref = S.triRef[prim];
-    const rtx_vertex &v0 = S.vertices[ref.y], &v1 = S.vertices[ref.z], &v2 = S.vertices[ref.w];
+    const float4 *ts = S.triShade + kTriShadeSlots * (size_t)prim;
+    const float4 v0 = ts[1], v1 = ts[3], v2 = ts[5];
     float b0 = 1.0f - bu - bv;
-    float u = v0.texCoord[0] * b0 + v1.texCoord[0] * bu + v2.texCoord[0] * bv;
-    float v = v0.texCoord[1] * b0 + v1.texCoord[1] * bu + v2.texCoord[1] * bv;
+    float u = v0.z * b0 + v1.z * bu + v2.z * bv;
+    float v = v0.w * b0 + v1.w * bu + v2.w * bv;
     Rng r{tea(satU32(u * 100000000.0f + ox * t), randomUInt)};
-    float alpha = texSample(S, S.materials[v0.materialIndex].textureIdDiffuse, u, v).w;
+    float alpha = texSample(S, S.materials[__float_as_int(ts[6].x)].textureIdDiffuse, u, v).w;
     return !(r.next() > alpha);
 }
 

@@ -17,7 +17,10 @@ namespace rtx {
 struct DevScene {
     const float4 *nodes;      // kWideNodeSlots x float4 per Bvh8Node
     const float4 *tris;       // 3 x float4 per triangle in leaf order: v0 (w = prim id bits), v1, v2
-    const int4 *triRef;       // per global triangle id: (instance, global indices of its three vertices)
+    // kTriShadeSlots x float4 per global triangle id, one 128-byte line: its
+    // vertices' (position, normal.x), (normal.y, normal.z, texture u, v) in
+    // model space, then (material, instance, the instance's iLight) as int bits
+    const float4 *triShade;
     const rtx_vertex *vertices;
     const uint32_t *indices;
     const uint32_t *vertexBase; // per model
@@ -25,7 +28,7 @@ struct DevScene {
     const rtx_instance *instances;
     const rtx_material *materials;
     const rtx_light *lights;
-    const int32_t *lightIndex;
+    const uint32_t *lightIndex; // the random light table: light | type << kLightTypeShift
     const rtx_face_sample *triTable;
     // Area-light sampling without the table -> index -> vertex -> material
     // chain: per face-table entry (light row x RTX_SIZE_TRI_RANDOM) the face's
@@ -38,8 +41,11 @@ struct DevScene {
     // the first: the primitive id), for MIS probe rays that look for their
     // light before they trace (FrameConst::probeFirstLight); lightFirstOk is
     // 0 when there are more than kProbeLightMax of them or one is
-    // alpha-tested (emissive spheres are found among `spheres`).
+    // alpha-tested.
     const float4 *lightTris;
+    const float4 *lightSpheres; // the emissive spheres: (centre, radius), in id order
+    const int32_t *lightSphereId;
+    uint32_t numLightSpheres;
     uint32_t numLightTris;
     uint32_t lightFirstOk;
     const rtx_sphere *spheres;
@@ -59,6 +65,8 @@ struct DevScene {
     const float *srgbToLinear;  // 256 entries
 };
 
+constexpr uint32_t kTriShadeSlots = 8;
+constexpr uint32_t kLightTypeShift = 28, kLightRowMask = (1u << kLightTypeShift) - 1u;
 constexpr size_t kEmitTableBytes = size_t(256) << 20;
 // Emissive triangles up to which probe rays look for their light first.
 constexpr uint32_t kProbeLightMax = 64;

@@ -60,19 +60,28 @@ RTX_DI void waveAppend2(bool a, uint32_t *ca, bool b, uint32_t *cb, int &ia, int
 }
 
 // One append of both the `a` and the `b` lanes, the b lanes behind the a
-// lanes: one atomic.
-RTX_DI void waveAppendBoth(bool a, bool b, uint32_t *counter, int &ia, int &ib) {
-    const uint64_t ma = __ballot(a), mb = __ballot(b);
-    const int lane = (int)__lane_id();
-    const uint32_t na = (uint32_t)__popcll(ma), nb = (uint32_t)__popcll(mb);
-    const int leader = (ma | mb) ? __ffsll((unsigned long long)(ma | mb)) - 1 : 0;
-    uint32_t base = 0;
-    if ((ma | mb) && lane == leader) base = atomicAdd(counter, na + nb);
-    base = __shfl(base, leader);
-    const uint64_t below = lane == 0 ? 0ull : ((~0ull) >> (64 - lane));
-    ia = a ? (int)(base + (uint32_t)__popcll(ma & below)) : -1;
-    ib = b ? (int)(base + na + (uint32_t)__popcll(mb & below)) : -1;
-}
+// lanes, with one atomic: issue() sends it and place() waits for it and gives
+// the slots (-1 for the other lanes), so that work between the two hides the
+// atomic's round trip to the memory side (1-2 us).
+struct WaveAppend {
+    uint64_t ma, mb;
+    uint32_t base;
+    RTX_DI void issue(bool a, bool b, uint32_t *counter) {
+        ma = __ballot(a);
+        mb = __ballot(b);
+        base = 0;
+        if ((ma | mb) && (int)__lane_id() == leader())
+            base = atomicAdd(counter, (uint32_t)(__popcll(ma) + __popcll(mb)));
+    }
+    RTX_DI int leader() const { return (ma | mb) ? __ffsll((unsigned long long)(ma | mb)) - 1 : 0; }
+    RTX_DI void place(int &ia, int &ib) const {
+        const int lane = (int)__lane_id();
+        const uint32_t first = __shfl(base, leader());
+        const uint64_t below = lane == 0 ? 0ull : ((~0ull) >> (64 - lane));
+        ia = (ma >> lane) & 1ull ? (int)(first + (uint32_t)__popcll(ma & below)) : -1;
+        ib = (mb >> lane) & 1ull ? (int)(first + (uint32_t)(__popcll(ma) + __popcll(mb & below))) : -1;
+    }
+};
 
 // Runs body(k) once for every distinct value k of `key` among the lanes
 // with `active`, with exactly the lanes holding that key active and k
@@ -357,8 +366,7 @@ RTX_DI V3 probeContribution(const DevScene &S, bool power, V3 o, V3 d, int prim,
     const rtx_material &ms = S.materials[hi.matIndex];
     if (ms.type != RTX_MAT_LIGHT) return v3(0.0f);
     emitter = true;
-    int iLight = hi.isSphere ? S.spheres[hi.instanceIndex].iLight : S.instances[hi.instanceIndex].iLight;
-    const rtx_light &light = S.lights[iLight];
+    const rtx_light &light = S.lights[hi.iLight];
     float cosL = dot(-d, hi.normal);
     float pdfL = light.sampleProb * t * t / cosL / light.area;
     float h = misWeight(power, pdfMat, pdfL);
@@ -376,12 +384,16 @@ RTX_DI int nearestLight(const DevScene &S, V3 o, V3 d, float tmin, float &tHit, 
     int best = -1;
     float tmax = kTMax;
     bu = bv = 0.0f;
-    for (uint32_t k = 0; k < S.numSpheres; ++k) {
-        const rtx_sphere &sp = S.spheres[k];
-        if (S.materials[sp.materialIndex].type != RTX_MAT_LIGHT) continue;
+    for (uint32_t k = 0; k < S.numLightSpheres; ++k) {
+        const float4 cr = S.lightSpheres[k];
+        const int id = S.lightSphereId[k];
+        rtx_sphere sp;
+        sp.center[0] = cr.x;
+        sp.center[1] = cr.y;
+        sp.center[2] = cr.z;
+        sp.radius = cr.w;
         float t;
         if (isectSphere(sp, r.o, r.d, tmin, tmax, t)) {
-            const int id = (int)(S.numTris + k);
             if (best < 0 || t < tmax || id < best) {
                 tmax = t;
                 best = id;
@@ -702,6 +714,36 @@ RTX_DI void pushSplit(const PathBuffers &pb, uint32_t pid, int4 &task, const Hit
 }
 
 // ----------------------------------------------------------------- shade
+// One NEE sample's rays and their places in the shadow and probe queues.
+struct NeeRays {
+    WaveAppend shadow, probe;
+    uint32_t slot;
+    V3 lightDir, bsdfDir;
+    float lightDist, occMax;
+    float4 probeBase;
+};
+RTX_DI void queueNee(const Queue &qs, const Queue &qp, V3 pos, const NeeRays &r, bool lightFirst) {
+    int si, oi, pi = -1, none;
+    r.shadow.place(si, oi);
+    if (!lightFirst) r.probe.place(pi, none);
+    if (si >= 0) {
+        qs.id[si] = (int)r.slot;
+        qs.org[si] = f4(pos, kTMin);
+        qs.dir[si] = f4(r.lightDir, r.lightDist * (1.0f - 0.0001f));
+    }
+    if (oi >= 0) {
+        qs.id[oi] = (int)r.slot | kProbeOccBit;
+        qs.org[oi] = f4(pos, kTMin);
+        qs.dir[oi] = f4(r.bsdfDir, r.occMax);
+    }
+    if (pi >= 0) {
+        qp.id[pi] = (int)r.slot;
+        qp.org[pi] = f4(pos, kTMin);
+        qp.dir[pi] = f4(r.bsdfDir, kTMax);
+        qp.aux[pi] = r.probeBase;
+    }
+}
+
 // Register budget: two waves per SIMD (at most 256 VGPRs), three for a cache
 // frame's two classes (at most 168; 44 cache frames' kShade2: 139 ms with two,
 // 134 with three, 142 with four, which spills 170 registers).  The plain build
@@ -817,6 +859,7 @@ RTX_DI void shadeLane(const DevScene &S, const DevIC &IC, const DevGuiding &G, c
             h.frontFace = (mf >> 31) != 0;
             h.isSphere = false;
             h.instanceIndex = 0;
+            h.iLight = -1;
             h.u = c.w;
             h.v = t.w;
             d = -v3(c);
@@ -969,6 +1012,7 @@ RTX_DI void shadeLane(const DevScene &S, const DevIC &IC, const DevGuiding &G, c
     const bool lightFirst = fc.probeFirstLight && S.lightFirstOk && S.env == nullptr;
     const V3 wi = -d;
     const V3 thrNee = thr; // the throughput NEE terms of this vertex carry
+    NeeRays neeRays; // of the last sample: queued once the continuation is done
     for (uint32_t j = 0; j < numNEE; ++j) {
         bool wantShadow = false, wantProbe = false, wantOcc = false;
         V3 lightDir = v3(0.0f), bsdfDir = v3(0.0f), probeBase = v3(0.0f);
@@ -1039,25 +1083,15 @@ RTX_DI void shadeLane(const DevScene &S, const DevIC &IC, const DevGuiding &G, c
         }
         // a light-first probe's occlusion ray goes to the shadow queue, behind
         // the wave's shadow rays; the other scenes' probes to their own
-        int si, pi = -1, oi = -1;
-        if (lightFirst) waveAppendBoth(wantShadow, wantOcc, &cnt->shadow.v, si, oi);
-        else waveAppend2(wantShadow, &cnt->shadow.v, wantProbe, &cnt->probe.v, si, pi);
-        if (wantOcc) {
-            qs.id[oi] = (int)slot | kProbeOccBit;
-            qs.org[oi] = f4(h.worldPos, kTMin);
-            qs.dir[oi] = f4(bsdfDir, occMax);
-        }
-        if (wantShadow) {
-            qs.id[si] = (int)slot;
-            qs.org[si] = f4(h.worldPos, kTMin);
-            qs.dir[si] = f4(lightDir, lightDist * (1.0f - 0.0001f));
-        }
-        if (wantProbe) {
-            qp.id[pi] = (int)slot;
-            qp.org[pi] = f4(h.worldPos, kTMin);
-            qp.dir[pi] = f4(bsdfDir, kTMax);
-            qp.aux[pi] = f4(probeBase, pdfMatProbe);
-        }
+        neeRays.slot = slot;
+        neeRays.lightDir = lightDir;
+        neeRays.lightDist = lightDist;
+        neeRays.bsdfDir = bsdfDir;
+        neeRays.occMax = occMax;
+        neeRays.probeBase = f4(probeBase, pdfMatProbe);
+        neeRays.shadow.issue(wantShadow, lightFirst && wantOcc, &cnt->shadow.v);
+        if (!lightFirst) neeRays.probe.issue(wantProbe, false, &cnt->probe.v);
+        if (j + 1 < numNEE) queueNee(qs, qp, h.worldPos, neeRays, lightFirst);
     }
     if (nrc) { // the learned cache's queries, in the order the waves reach them
         const int qn = waveAppend(nrcQ, pb.nrcQueryCount);
@@ -1155,6 +1189,7 @@ RTX_DI void shadeLane(const DevScene &S, const DevIC &IC, const DevGuiding &G, c
             pb.grec[pid] = grec;
         }
     }
+    if (numNEE > 0) queueNee(qs, qp, h.worldPos, neeRays, lightFirst);
     int qi, di;
     waveAppend2(cont, nextCount, isDone, &cnt->done[qsel].v, qi, di);
     if (cont) {
