@@ -993,6 +993,8 @@ int rtx_render(rtx_ctx *ctx, const rtx_scene *scene, const rtx_frame_params *p, 
             CHECK_HIP(ctx, devAlloc(&ctx->pb.nrcQueryAux, bufPaths, L));
             CHECK_HIP(ctx, devAlloc(&ctx->pb.nrcPath, 2 * bufPaths, L));
             CHECK_HIP(ctx, devAlloc(&ctx->pb.nrcQueryCount, 1, L));
+            CHECK_HIP(ctx, devAlloc(&ctx->nrcFeat, (size_t)kNrcMaxLevels * std::min(bufPaths, kNrcInferRows), L));
+            ctx->pb.nrcQueryStride = (uint32_t)bufPaths;
             ctx->nrcPathCap = bufPaths;
         }
         nrcEvery = (uint32_t)std::max<uint64_t>(1, npix / ctx->nrcCfg.trainingPaths);
@@ -1255,7 +1257,8 @@ int rtx_render(rtx_ctx *ctx, const rtx_scene *scene, const rtx_frame_params *p, 
             if (rcb != RTX_OK) return rcb;
             if (nrc) // the paths that ended into the learned cache: throughput x cache
                 timed(kClsShade, [&] {
-                    launchNrcInfer(s, ctx->nrc, ctx->pb.nrcQuery, b.numPaths, ctx->pb.nrcQueryCount, nullptr,
+                    launchNrcInfer(s, ctx->nrc, ctx->pb.nrcQuery, NrcRows{1, ctx->pb.nrcQueryStride}, b.numPaths,
+                                   ctx->pb.nrcQueryCount, ctx->nrcFeat, nullptr,
                                    ctx->pb.nrcQueryAux, ctx->pb.out, 2 * ctx->cuCount,
                                    NrcSelfTrain{ctx->pb.thr, ctx->pb.nrcPath,
                                                 fc.nrcSuffix ? ctx->pb.nrcTrainTarget : nullptr, kFlagNrcTrainEnd});
@@ -2011,6 +2014,8 @@ static void nrcFree(rtx_ctx *ctx) {
     ctx->nrcPathCap = ctx->nrcSlotCap = 0;
     ctx->pb.nrcQuery = ctx->pb.nrcQueryAux = ctx->pb.nrcPath = nullptr;
     ctx->pb.nrcQueryCount = nullptr;
+    ctx->pb.nrcQueryStride = 0;
+    ctx->nrcFeat = nullptr;
     ctx->pb.nrcTrainIn = ctx->pb.nrcTrainTarget = nullptr;
 }
 
@@ -2130,6 +2135,7 @@ int rtx_nrc_create(rtx_ctx *ctx, const rtx_nrc_config *c) try {
         nb.gridBf16Ema = nb.gridBf16;
         nb.wFwdEma = nb.wFwd;
     }
+    CHECK_HIP(ctx, devAlloc(&nb.feat, (size_t)kNrcMaxLevels * nb.rowsCap, L));
     CHECK_HIP(ctx, devAlloc(&nb.acts, (size_t)kNrcLayers * nb.rowsCap * 64, L));
     CHECK_HIP(ctx, devAlloc(&nb.dz, (size_t)kNrcLayers * nb.rowsCap * 64, L));
     CHECK_HIP(ctx, devAlloc(&nb.pred, (size_t)nb.rowsCap * 4, L));
@@ -2261,11 +2267,14 @@ int rtx_nrc_infer(rtx_ctx *ctx, const rtx_nrc_input *in, size_t n, float *rgb) t
     CHECK_HIP(ctx, hipSetDevice(ctx->device));
     std::vector<void *> tmp;
     float4 *inD = nullptr, *outD = nullptr;
+    uint32_t *feat = nullptr;
     int rc = nrcUpload(ctx, in, nullptr, n, tmp, &inD, nullptr);
     if (rc == RTX_OK) {
         hipError_t e = devAlloc(&outD, n, tmp);
+        if (e == hipSuccess) e = devAlloc(&feat, (size_t)kNrcMaxLevels * std::min(n, kNrcInferRows), tmp);
         if (e == hipSuccess) {
-            launchNrcInfer(ctx->stream, ctx->nrc, inD, (uint32_t)n, nullptr, outD, nullptr, nullptr, 2 * ctx->cuCount);
+            launchNrcInfer(ctx->stream, ctx->nrc, inD, NrcRows{4, 1}, (uint32_t)n, nullptr, feat, outD, nullptr,
+                           nullptr, 2 * ctx->cuCount);
             e = hipGetLastError();
         }
         std::vector<float4> out(n);

@@ -125,6 +125,7 @@ struct rtx_ctx {
     rtx_nrc_config nrcCfg{};
     NrcBuffers nrc{};
     std::vector<void *> nrcAllocs, nrcPathAllocs, nrcSlotAllocs;
+    uint32_t *nrcFeat = nullptr; // in nrcPathAllocs: the encoded features of a batch's queries
     float *nrcLoss = nullptr;   // device: summed loss of the last steps
     uint32_t nrcLossSteps = 0;
     size_t nrcPathCap = 0, nrcSlotCap = 0;

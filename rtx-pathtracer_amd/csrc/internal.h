@@ -308,12 +308,14 @@ struct PathBuffers {
                       // (wi, texture u), (throughput, texture v)  (splitInfo, raytrace.rgen:70-80)
     const float4 *estimate; // per pixel: the ADRRS estimate (estimateImage)
     uint32_t *frameSeed;    // per path: the frame's randomUInt (any-hit alpha test seeds)
-    // learned radiance cache: the queries of paths that end into it (4 float4
-    // of rtx_nrc_input each; aux = (throughput, path id bits)), training
+    // learned radiance cache: the queries of paths that end into it (the 4
+    // float4 of an rtx_nrc_input in arrays nrcQueryStride apart, so that a
+    // wave's stores and the cache's reads are coalesced; aux = (throughput, path id bits)), training
     // vertices by slot (input, and target rgb with w = 1 once the path ended),
     // and per path (throughput at the training vertex, slot bits), (radiance so far)
     float4 *nrcQuery, *nrcQueryAux;
     uint32_t *nrcQueryCount;
+    uint32_t nrcQueryStride;
     float4 *nrcTrainIn, *nrcTrainTarget;
     float4 *nrcPath;
 };

@@ -1099,11 +1099,12 @@ RTX_DI void shadeLane(const DevScene &S, const DevIC &IC, const DevGuiding &G, c
             float rough;
             V3 alb;
             nrcSurface(m, rough, alb);
-            float4 *q = pb.nrcQuery + 4 * (size_t)qn;
+            const size_t stride = pb.nrcQueryStride;
+            float4 *q = pb.nrcQuery + qn;
             q[0] = f4(h.worldPos, rough);
-            q[1] = f4(-d, 0.0f);
-            q[2] = f4(h.normal, 0.0f);
-            q[3] = f4(alb, 0.0f);
+            q[stride] = f4(-d, 0.0f);
+            q[2 * stride] = f4(h.normal, 0.0f);
+            q[3 * stride] = f4(alb, 0.0f);
             pb.nrcQueryAux[qn] = f4(thr, __uint_as_float(pid));
         }
     }

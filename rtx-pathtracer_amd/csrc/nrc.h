@@ -53,6 +53,7 @@ struct NrcBuffers {
     uint16_t *wFwdEma;
     float emaDecay;
     // training batch work (rows = trainBatch)
+    uint32_t *feat;             // [16][rows]: the encoded features, two bf16 a level
     uint16_t *acts;             // [6][rows][64] bf16: the input of every layer
     uint16_t *dz;               // [6][rows][64] bf16: d loss / d pre-activation of every layer
     float *pred;                // [rows][4]
@@ -61,6 +62,14 @@ struct NrcBuffers {
     uint32_t rowsCap;
     uint32_t step;              // Adam steps taken
     float lr, beta1, beta2, eps;
+};
+
+// Where row r's field k (0: position and roughness, 1: direction, 2: normal,
+// 3: albedo; a float4 each) is: rtx_nrc_input records one after another, or
+// each field in an array of its own.
+struct NrcRows {
+    size_t row, field;
+    __host__ __device__ size_t at(size_t r, size_t k) const { return r * row + k * field; }
 };
 
 // Self-training suffixes (inference inside a render): a query whose path has
@@ -72,9 +81,14 @@ struct NrcSelfTrain {
     float4 *target;   // NULL: no self-training
     uint32_t endFlag;
 };
-// n rows, or *count rows (at most n) when count is given
-void launchNrcInfer(hipStream_t s, const NrcBuffers &nb, const float4 *in, uint32_t n, const uint32_t *count,
-                    float4 *out, const float4 *aux, float4 *pathOut, int blocks, NrcSelfTrain st = NrcSelfTrain{});
+// Inference encodes and evaluates at most this many rows at a time, which
+// bounds the features between the two kernels (256 MB).
+constexpr size_t kNrcInferRows = 1u << 22;
+// n rows, or *count rows (at most n) when count is given; feat: work memory,
+// kNrcMaxLevels x min(n, kNrcInferRows) words
+void launchNrcInfer(hipStream_t s, const NrcBuffers &nb, const float4 *in, NrcRows rows, uint32_t n,
+                    const uint32_t *count, uint32_t *feat, float4 *out, const float4 *aux, float4 *pathOut, int blocks,
+                    NrcSelfTrain st = {});
 // Rows (queries, training vertices) are rtx_nrc_input records, 4 float4 each:
 // (pos, roughness), (dir, -), (normal, -), (albedo, -).
 // Forward with saved activations, the loss gradient, the backward pass, the

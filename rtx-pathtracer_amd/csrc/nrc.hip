@@ -1,4 +1,4 @@
-// Learned radiance cache kernels: hash-grid encoding, the fused 5 x 64 MLP on
+// Learned radiance cache kernels: hash-grid encoding, the 5 x 64 MLP on
 // BF16 MFMA (v_mfma_f32_16x16x32_bf16, FP32 accumulation), its backward
 // pass, weight and grid gradients, and Adam.
 //
@@ -28,6 +28,7 @@ constexpr int kBlock = 256;       // 4 waves
 constexpr int kRowsPerWave = 32;
 constexpr int kChunk = 256;       // batch rows per weight-gradient workgroup
 constexpr int kChunkPitch = kChunk + 8;
+constexpr uint32_t kEncodeChunks = 512; // blocks per XCD: 16 each for its 32 CUs, which holds 8 (2 passes)
 constexpr int kWLayer = kNrcWidth * kNrcWidth; // bf16 per layer in the packed weight arrays
 
 __device__ __forceinline__ uint16_t f2bf(float x) { return __builtin_bit_cast(uint16_t, (__bf16)x); }
@@ -37,32 +38,44 @@ __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// Hash-grid lookup of level l at the normalised position p: the trilinear
-// blend of the 8 surrounding entries' two features.  Dense levels index
-// x + (res+1)(y + (res+1) z); finer levels hash with the primes of Teschner
-// et al. (2003) as instant-ngp does.  No contraction, so the weights and sums
-// round the same way as a plain restatement.
-__device__ void gridCorner(const NrcGrid &g, int l, const float p[3], int c, uint32_t &idx, float &w) {
+// The cell of level l that holds the normalised position p: its lower corner
+// and the position within it.  No contraction anywhere in the encoding, so the
+// weights and sums round the same way as a plain restatement.
+struct GridCell {
+    uint32_t lo[3];
+    float t[3];
+};
+__device__ __forceinline__ GridCell gridCell(const NrcGrid &g, int l, const float p[3]) {
 #pragma clang fp contract(off)
     const float r = g.res[l];
-    uint32_t ci[3];
-    float wt = 1.0f;
+    GridCell c;
+#pragma unroll
     for (int a = 0; a < 3; ++a) {
         const float x = p[a] * r;
         float f = fminf(floorf(x), r - 1.0f);
         f = fmaxf(f, 0.0f);
-        const float t = x - f;
-        const uint32_t bit = (uint32_t)(c >> a) & 1u;
-        ci[a] = (uint32_t)f + bit;
-        wt = wt * (bit ? t : 1.0f - t);
+        c.t[a] = x - f;
+        c.lo[a] = (uint32_t)f;
     }
+    return c;
+}
+// The table index of corner (x, y, z): dense levels index x + (res + 1)
+// (y + (res + 1) z); finer levels hash with the primes of Teschner et al.
+// (2003) as instant-ngp does.
+__device__ __forceinline__ uint32_t gridIndex(const NrcGrid &g, int l, uint32_t x, uint32_t y, uint32_t z) {
     if (g.dense[l]) {
-        const uint32_t n1 = (uint32_t)r + 1u;
-        idx = ci[0] + n1 * (ci[1] + n1 * ci[2]);
-    } else {
-        idx = (ci[0] ^ (ci[1] * 2654435761u) ^ (ci[2] * 805459861u)) & g.tableMask;
+        const uint32_t n1 = (uint32_t)g.res[l] + 1u;
+        return x + n1 * (y + n1 * z);
     }
-    w = wt;
+    return (x ^ (y * 2654435761u) ^ (z * 805459861u)) & g.tableMask;
+}
+// The trilinear weight of corner c (bit a of c: the upper side on axis a).
+__device__ __forceinline__ float cornerWeight(const GridCell &cell, int c) {
+#pragma clang fp contract(off)
+    float wt = 1.0f;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) wt = wt * ((c >> a) & 1 ? cell.t[a] : 1.0f - cell.t[a]);
+    return wt;
 }
 
 __device__ void normalisedPos(const NrcGrid &g, float4 in0, float p[3]) {
@@ -72,56 +85,107 @@ __device__ void normalisedPos(const NrcGrid &g, float4 in0, float p[3]) {
     p[2] = fminf(fmaxf((in0.z - g.lo[2]) * g.inv[2], 0.0f), 1.0f);
 }
 
-__device__ void encodeLevel(const NrcGrid &g, const uint32_t *table, int l, const float p[3], float &f0, float &f1) {
+// Two neighbouring entries along x, in one 8-byte load where they share one:
+// always in a dense level (consecutive entries), and in a hashed level when x
+// is even, since the hash then differs in its lowest bit alone.
+struct __attribute__((packed, aligned(4))) EntryPair {
+    uint32_t a, b;
+};
+__device__ __forceinline__ void loadPair(const NrcGrid &g, const uint32_t *tab, int l, uint32_t x, uint32_t y,
+                                         uint32_t z, uint32_t &lo, uint32_t &hi) {
+    const uint32_t i = gridIndex(g, l, x, y, z);
+    if (g.dense[l]) {
+        const EntryPair e = *reinterpret_cast<const EntryPair *>(tab + i);
+        lo = e.a;
+        hi = e.b;
+        return;
+    }
+    const uint2 e = *reinterpret_cast<const uint2 *>(tab + (i & ~1u));
+    lo = i & 1u ? e.y : e.x;
+    hi = i & 1u ? e.x : e.y;
+    if (x & 1u) hi = tab[gridIndex(g, l, x + 1u, y, z)];
+}
+
+// The rows of a launch: n of them, or as many of the *count (when count is
+// given) as lie past the first `first`.
+struct NrcRange {
+    uint32_t n;
+    const uint32_t *count;
+    uint32_t first;
+    __device__ uint32_t rows() const { return count ? min(max(*count, first) - first, n) : n; }
+};
+
+// The hash-grid features of rows [0, n): for level l the trilinear blend of the
+// 8 surrounding entries' two features, packed bf16, to feat[l * stride + row].
+// Blocks are dispatched to the 8 XCDs in turn, and each XCD encodes two levels
+// (blockIdx % 8 and 8 more) of every row: two levels' tables are 4 MB, which
+// is an XCD's L2 (97% hits), where all 16 levels' 33 MB missed it on most of a
+// row's 128 gathers.  A row's thread has its 8 corners' loads in flight at
+// once, and pairs of them share a load (loadPair: 86 loads a row instead of
+// 128).  What bounds it now is the lines from L2 to the L1s, one per load and
+// lane (address units 77% busy).  1.9 M queries of a frame, default tables:
+// 1.34 ms encoded and evaluated in one kernel; 0.76 ms here and 0.25 ms in
+// kNrcForward.  Loads past L1 are no faster, non-temporal ones 1.19 ms.
+__global__ __launch_bounds__(256) void kNrcEncode(NrcGrid g, const uint32_t *table, const float4 *in,
+                                                  NrcRows rows, NrcRange range, uint32_t *feat, size_t stride) {
 #pragma clang fp contract(off)
-    const uint32_t *tab = table + (size_t)l * (g.tableMask + 1u);
-    f0 = 0.0f;
-    f1 = 0.0f;
-    for (int c = 0; c < 8; ++c) {
-        uint32_t idx;
-        float w;
-        gridCorner(g, l, p, c, idx, w);
-        const uint32_t v = tab[idx];
-        f0 = f0 + w * bf2f(v & 0xFFFFu);
-        f1 = f1 + w * bf2f(v >> 16);
+    const uint32_t n = range.rows();
+    const uint32_t step = (gridDim.x >> 3) * 256u;
+    for (uint32_t row = (blockIdx.x >> 3) * 256u + threadIdx.x; row < n; row += step) {
+        float p[3];
+        normalisedPos(g, in[rows.at(row, 0)], p);
+        for (int l = blockIdx.x & 7; l < (int)g.levels; l += 8) {
+            const uint32_t *tab = table + (size_t)l * (g.tableMask + 1u);
+            const GridCell cell = gridCell(g, l, p);
+            uint32_t v[8];
+#pragma unroll
+            for (int c = 0; c < 8; c += 2)
+                loadPair(g, tab, l, cell.lo[0], cell.lo[1] + ((c >> 1) & 1), cell.lo[2] + (c >> 2), v[c], v[c + 1]);
+            float f0 = 0.0f, f1 = 0.0f;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                const float w = cornerWeight(cell, c);
+                f0 = f0 + w * bf2f(v[c] & 0xFFFFu);
+                f1 = f1 + w * bf2f(v[c] >> 16);
+            }
+            feat[l * stride + row] = (uint32_t)f2bf(f0) | (uint32_t)f2bf(f1) << 16;
+        }
     }
 }
 
 // The network input of rows [row0, row0 + 128) into the block's activation
-// tile (bf16, row-major, kPitch): 2 features per level, then direction,
+// tile (bf16, row-major, kPitch): the encoded features, then direction,
 // normal, roughness, albedo, a constant 1 (the layers have no bias) and
 // zeros.  Rows past n are all zero.
-__device__ void encodeTile(const NrcGrid &g, const uint32_t *table, const float4 *in, uint32_t row0, uint32_t n,
-                           uint16_t *act) {
+__device__ void loadTile(const NrcGrid &g, const uint32_t *feat, size_t stride, const float4 *in, NrcRows rows,
+                         uint32_t row0, uint32_t n, uint16_t *act) {
     const int t = threadIdx.x;
     const int r = t & (kNrcRowsPerBlock - 1);
     const uint32_t row = row0 + (uint32_t)r;
     const bool valid = row < n;
-    uint16_t *dst = act + r * kPitch;
-    float p[3] = {0.0f, 0.0f, 0.0f};
-    float4 in0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    if (valid) {
-        in0 = in[4 * (size_t)row];
-        normalisedPos(g, in0, p);
+    uint32_t *dst = reinterpret_cast<uint32_t *>(act + r * kPitch); // two values a word
+    uint32_t f[kNrcMaxLevels / 2];
+#pragma unroll
+    for (int k = 0; k < kNrcMaxLevels / 2; ++k) {
+        const int l = (t >> 7) + 2 * k;
+        f[k] = valid && l < (int)g.levels ? feat[l * stride + row] : 0u;
     }
-    for (int l = t >> 7; l < kNrcMaxLevels; l += 2) {
-        float f0 = 0.0f, f1 = 0.0f;
-        if (valid && l < (int)g.levels) encodeLevel(g, table, l, p, f0, f1);
-        dst[2 * l] = f2bf(f0);
-        dst[2 * l + 1] = f2bf(f1);
-    }
+#pragma unroll
+    for (int k = 0; k < kNrcMaxLevels / 2; ++k) dst[(t >> 7) + 2 * k] = f[k];
     if (t < kNrcRowsPerBlock) {
         float v[32];
         for (int k = 0; k < 32; ++k) v[k] = 0.0f;
         if (valid) {
-            const float4 a = in[4 * (size_t)row + 1], b = in[4 * (size_t)row + 2], c = in[4 * (size_t)row + 3];
+            const float4 in0 = in[rows.at(row, 0)], a = in[rows.at(row, 1)], b = in[rows.at(row, 2)],
+                         c = in[rows.at(row, 3)];
             v[0] = a.x, v[1] = a.y, v[2] = a.z;   // direction
             v[3] = b.x, v[4] = b.y, v[5] = b.z;   // normal
             v[6] = in0.w;                         // roughness
             v[7] = c.x, v[8] = c.y, v[9] = c.z;   // albedo
             v[10] = 1.0f;
         }
-        for (int k = 0; k < 32; ++k) dst[32 + k] = f2bf(v[k]);
+#pragma unroll
+        for (int k = 0; k < 32; k += 2) dst[16 + k / 2] = (uint32_t)f2bf(v[k]) | (uint32_t)f2bf(v[k + 1]) << 16;
     }
 }
 
@@ -180,14 +244,15 @@ __device__ void mlpWave(const uint16_t *wf, uint16_t *act, uint16_t *acts, uint3
 // Rows are queries (4 float4 of input each).  out (optional): the raw RGB
 // prediction per row.  pathOut (optional): the render's per-path radiance,
 // to which max(prediction, 0) times the query's throughput aux[row].xyz is
-// added for path aux[row].w.  n = *count when count is given.
+// added for path aux[row].w.
 template <bool TRAIN>
-__global__ __launch_bounds__(kBlock) void kNrcForward(NrcBuffers nb, const float4 *in, uint32_t nHost,
-                                                      const uint32_t *count, float4 *out, const float4 *aux,
-                                                      float4 *pathOut, NrcSelfTrain st) {
+__global__ __launch_bounds__(kBlock) void kNrcForward(NrcBuffers nb, const uint32_t *feat, size_t stride,
+                                                      const float4 *in, NrcRows rows, NrcRange range,
+                                                      float4 *out, const float4 *aux, float4 *pathOut,
+                                                      NrcSelfTrain st) {
     __shared__ __align__(16) uint16_t wf[kNrcLayers * kNrcWidth * kPitch];
     __shared__ __align__(16) uint16_t act[kNrcRowsPerBlock * kPitch];
-    const uint32_t n = count ? min(*count, nHost) : nHost;
+    const uint32_t n = range.rows();
     // training runs whole 256-row chunks (rows past n are zeros), inference n rows
     const uint32_t rowsEnd = TRAIN ? ((n + 255u) & ~255u) : n;
     if ((uint32_t)blockIdx.x * kNrcRowsPerBlock >= rowsEnd) return;
@@ -197,7 +262,7 @@ __global__ __launch_bounds__(kBlock) void kNrcForward(NrcBuffers nb, const float
     float *scratch = reinterpret_cast<float *>(wact); // 32 rows x 4 floats after the last layer
     for (uint32_t row0 = blockIdx.x * kNrcRowsPerBlock; row0 < rowsEnd; row0 += gridDim.x * kNrcRowsPerBlock) {
         __syncthreads(); // the previous tile's readers are done with act
-        encodeTile(nb.grid, nb.gridBf16, in, row0, n, act);
+        loadTile(nb.grid, feat, stride, in, rows, row0, n, act);
         __syncthreads();
         f32x4 o[2];
         const uint32_t wrow0 = row0 + wave * kRowsPerWave;
@@ -361,36 +426,42 @@ __global__ __launch_bounds__(kBlock) void kNrcWeightGrad(NrcBuffers nb) {
 }
 
 // Sums the partials of every chunk in chunk order into the MLP gradients
-// (out-major, after the grid's parameters).
+// (out-major, after the grid's parameters).  Threads follow the partials'
+// order, [in][out], so that the many reads are the coalesced side, with eight
+// in flight: 37.5 us for 64 chunks, 10 us so.
 __global__ __launch_bounds__(256) void kNrcReduceGrad(NrcBuffers nb, uint32_t chunks) {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= (uint32_t)kNrcMlpParams) return;
+    if (i >= (uint32_t)(kNrcLayers * kNrcWidth * kNrcWidth)) return;
     const uint32_t layer = i / (kNrcWidth * kNrcWidth), rem = i % (kNrcWidth * kNrcWidth);
-    const uint32_t o = rem / kNrcWidth, k = rem % kNrcWidth;
+    const uint32_t k = rem / kNrcWidth, o = rem % kNrcWidth;
     if (layer == kNrcLayers - 1 && o >= 3) return; // padding rows of the output layer stay zero
     float s = 0.0f;
+#pragma unroll 8
     for (uint32_t c = 0; c < chunks; ++c)
-        s += nb.partials[((size_t)c * kNrcLayers + layer) * (kNrcWidth * kNrcWidth) + k * kNrcWidth + o];
-    nb.grads[nb.gridParams + i] += s;
+        s += nb.partials[((size_t)c * kNrcLayers + layer) * (kNrcWidth * kNrcWidth) + rem];
+    nb.grads[nb.gridParams + layer * (kNrcWidth * kNrcWidth) + o * kNrcWidth + k] += s;
 }
 
 // d loss / d table entries: each row's feature gradients spread over the 8
-// corners of every level with the trilinear weights (FP32 atomics).
+// corners of every level with the trilinear weights (FP32 atomics).  The
+// atomics bound it, and the memory side takes them by requests, one per line
+// and instruction: 16 lanes share a row (feature, then x, y, z of the corner),
+// so that an entry's two sums, and two entries next to each other along x
+// (always in a dense level, in a hashed one from an even x), go as one.
+// 16,384 rows: 245 us with a lane per row and level and 16 atomics each, 72 us so.
 __global__ __launch_bounds__(256) void kNrcGridGrad(NrcBuffers nb, const float4 *in, uint32_t n) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    const uint32_t row = i / kNrcMaxLevels, l = i % kNrcMaxLevels;
-    if (row >= n || l >= nb.grid.levels) return;
-    float p[3];
-    normalisedPos(nb.grid, in[4 * (size_t)row], p);
-    const float g0 = nb.dFeat[(size_t)row * 32 + 2 * l], g1 = nb.dFeat[(size_t)row * 32 + 2 * l + 1];
-    if (g0 == 0.0f && g1 == 0.0f) return;
-    float *gg = nb.grads + (size_t)l * (nb.grid.tableMask + 1u) * 2;
-    for (int c = 0; c < 8; ++c) {
-        uint32_t idx;
-        float w;
-        gridCorner(nb.grid, (int)l, p, c, idx, w);
-        atomicAdd(gg + 2 * (size_t)idx, w * g0);
-        atomicAdd(gg + 2 * (size_t)idx + 1, w * g1);
+    const int feature = threadIdx.x & 1, c = (threadIdx.x >> 1) & 7;
+    for (uint32_t row = blockIdx.x * 16u + (threadIdx.x >> 4); row < n; row += gridDim.x * 16u) {
+        float p[3];
+        normalisedPos(nb.grid, in[4 * (size_t)row], p);
+        for (uint32_t l = 0; l < nb.grid.levels; ++l) {
+            const float d = nb.dFeat[(size_t)row * 32 + 2 * l + feature];
+            if (d == 0.0f) continue;
+            const GridCell cell = gridCell(nb.grid, l, p);
+            const uint32_t idx = gridIndex(nb.grid, l, cell.lo[0] + (c & 1), cell.lo[1] + ((c >> 1) & 1),
+                                           cell.lo[2] + (c >> 2));
+            atomicAdd(nb.grads + ((size_t)l * (nb.grid.tableMask + 1u) + idx) * 2 + feature, cornerWeight(cell, c) * d);
+        }
     }
 }
 
@@ -453,15 +524,29 @@ __global__ __launch_bounds__(256) void kNrcZero(float *p, size_t n) {
 
 } // namespace
 
-void launchNrcInfer(hipStream_t s, const NrcBuffers &nb, const float4 *in, uint32_t n, const uint32_t *count,
-                    float4 *out, const float4 *aux, float4 *pathOut, int blocks, NrcSelfTrain st) {
-    if (n == 0) return;
-    const int tiles = (int)((n + kNrcRowsPerBlock - 1) / kNrcRowsPerBlock);
+// A multiple of 8 blocks: every XCD sees all rows.
+static void launchEncode(hipStream_t s, const NrcBuffers &nb, const float4 *in, NrcRows rows, NrcRange range,
+                         uint32_t *feat, size_t stride) {
+    const uint32_t chunks = (range.n + 255u) / 256u;
+    hipLaunchKernelGGL(kNrcEncode, dim3(8u * (chunks < kEncodeChunks ? chunks : kEncodeChunks)), dim3(256), 0, s,
+                       nb.grid, nb.gridBf16, in, rows, range, feat, stride);
+}
+
+void launchNrcInfer(hipStream_t s, const NrcBuffers &nb, const float4 *in, NrcRows rows, uint32_t n,
+                    const uint32_t *count, uint32_t *feat, float4 *out, const float4 *aux, float4 *pathOut, int blocks,
+                    NrcSelfTrain st) {
     NrcBuffers v = nb; // inference reads the moving average's copies
     v.gridBf16 = nb.gridBf16Ema;
     v.wFwd = nb.wFwdEma;
-    hipLaunchKernelGGL(kNrcForward<false>, dim3(tiles < blocks ? tiles : blocks), dim3(kBlock), 0, s, v, in, n,
-                       count, out, aux, pathOut, st);
+    const size_t stride = n < kNrcInferRows ? n : kNrcInferRows;
+    for (size_t r0 = 0; r0 < n; r0 += stride) {
+        const NrcRange range{(uint32_t)(n - r0 < stride ? n - r0 : stride), count, (uint32_t)r0};
+        const int tiles = (int)((range.n + kNrcRowsPerBlock - 1) / kNrcRowsPerBlock);
+        const float4 *rin = in + rows.at(r0, 0);
+        launchEncode(s, v, rin, rows, range, feat, stride);
+        hipLaunchKernelGGL(kNrcForward<false>, dim3(tiles < blocks ? tiles : blocks), dim3(kBlock), 0, s, v, feat,
+                           stride, rin, rows, range, out ? out + r0 : nullptr, aux ? aux + r0 : nullptr, pathOut, st);
+    }
 }
 
 void launchNrcGradients(hipStream_t s, NrcBuffers nb, const float4 *in, const float4 *target, uint32_t n,
@@ -471,13 +556,15 @@ void launchNrcGradients(hipStream_t s, NrcBuffers nb, const float4 *in, const fl
     // so the weight gradients' last chunk reads zeros, not stale rows
     const uint32_t chunks = (n + kChunk - 1) / kChunk;
     const uint32_t tiles = chunks * (kChunk / kNrcRowsPerBlock);
-    hipLaunchKernelGGL(kNrcForward<true>, dim3(tiles), dim3(kBlock), 0, s, nb, in, n, (const uint32_t *)nullptr,
-                       (float4 *)nullptr, (const float4 *)nullptr, (float4 *)nullptr, NrcSelfTrain{});
+    const NrcRows rows{4, 1};
+    const NrcRange range{n, nullptr, 0};
+    launchEncode(s, nb, in, rows, range, nb.feat, nb.rowsCap);
+    hipLaunchKernelGGL(kNrcForward<true>, dim3(tiles), dim3(kBlock), 0, s, nb, nb.feat, (size_t)nb.rowsCap, in, rows,
+                       range, (float4 *)nullptr, (const float4 *)nullptr, (float4 *)nullptr, NrcSelfTrain{});
     hipLaunchKernelGGL(kNrcBackward, dim3(tiles), dim3(kBlock), 0, s, nb, target, n, invCount, lossOut);
     hipLaunchKernelGGL(kNrcWeightGrad, dim3(chunks, kNrcLayers), dim3(kBlock), 0, s, nb);
-    hipLaunchKernelGGL(kNrcReduceGrad, dim3((kNrcMlpParams + 255) / 256), dim3(256), 0, s, nb, chunks);
-    const uint32_t pairs = n * kNrcMaxLevels;
-    hipLaunchKernelGGL(kNrcGridGrad, dim3((pairs + 255) / 256), dim3(256), 0, s, nb, in, n);
+    hipLaunchKernelGGL(kNrcReduceGrad, dim3(kNrcLayers * kNrcWidth * kNrcWidth / 256), dim3(256), 0, s, nb, chunks);
+    hipLaunchKernelGGL(kNrcGridGrad, dim3(16u * chunks), dim3(256), 0, s, nb, in, n);
     (void)cuCount;
 }
 
