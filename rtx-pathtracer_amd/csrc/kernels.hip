@@ -799,10 +799,11 @@ RTX_DI void shadeLane(const DevScene &S, const DevIC &IC, const DevGuiding &G, c
     int depth = 0, followCount = 0;
     bool follow = false, addNext = false, icHit = false;
     bool splitV = false, pendTask = false, dead = false, taskDirty = false, nrcQ = false;
+    bool vertex = false, nee = false, wantIC = false; // a vertex with a continuous BSDF; its NEE; its cache lookup
     int4 task = make_int4(0, 0, 0, 0); // (camera samples left, splits queued, next split, record sampleOffset)
     uint32_t ncand = 0;
     int4 grec = make_int4(0, -1, 0, 0); // record state: slot, distance slot, distanceFactor bits, NEE base
-    float firstT = kTMax;
+    float firstT = kTMax, hitT = 0.0f;
     if (active) {
         const uint32_t raw = (uint32_t)qin.id[i];
         splitV = (F & kShadeSegments) && (raw & kSplitVertex) != 0;
@@ -892,6 +893,7 @@ RTX_DI void shadeLane(const DevScene &S, const DevIC &IC, const DevGuiding &G, c
             }
             isDone = true;
         } else {
+            hitT = hit.x;
             if (depth == 1) firstT = hit.x;
 #ifdef RTX_DEVICE_DEBUG
             if (b.firstPath + (pid - b.pathBase) == fc.debugPath)
@@ -911,7 +913,8 @@ RTX_DI void shadeLane(const DevScene &S, const DevIC &IC, const DevGuiding &G, c
             } else {
                 addNext = false;
                 follow = false;
-                bool nee = useNEE;
+                vertex = true;
+                nee = useNEE;
                 if (nrc && depth >= (int)fc.nrcDepth && !(flags & kFlagNrcTrain)) {
                     const int slot = nrcSlot(fc, b, pid);
                     if (slot < 0) { // the path ends into the learned cache here, without NEE
@@ -942,66 +945,76 @@ RTX_DI void shadeLane(const DevScene &S, const DevIC &IC, const DevGuiding &G, c
                         flags |= kFlagNrcTrainEnd;
                     }
                 }
-                if ((useIC || (useADRRS && depth > 1)) && isICCapable(m.type, icOnGlossy)) { // raytrace.rgen:1080-1139
-                    V3 irr;
-                    if (icQuery(IC, icp, h.worldPos, h.normal, irr)) {
-                        if (useADRRS) { // weight window against the cache's irradiance (1087-1116)
-                            const uint32_t pixel = (uint32_t)((b.firstPath + (pid - b.pathBase)) % b.npix);
-                            int nw;
-                            float q = weightWindow(rng, v3(pb.estimate[pixel]), irr, thr, adrrsS, nw);
-                            if (nw == 1) {
-                                if (rng.next() > q) { // the path dies here, before its NEE
-                                    hash = sigFold(hash, kSigRRKill);
-                                    dead = true;
-                                } else {
-                                    thr = thr / q;
-                                }
-                            } else if (adrrsSplit) {
-                                const int room = kMaxSplits - task.y;
-                                if (nw - 1 > room) {
-                                    nw = room + 1;
-                                    q = (float)nw;
-                                }
-                                thr = thr / q;
-                                for (int k = 0; k < nw - 1; ++k) pushSplit(pb, pid, task, h, -d, thr, depth);
-                                taskDirty = true;
-                                hash = sigFold(hash, kSigSplit ^ (uint32_t)(nw - 1));
-                            }
-                        } else {
-                            // a cache record ends the path after its NEE (1114-1122)
-                            hash = sigFold(hash, kSigCacheHit);
-                            res = res + thr * approxDiffuse(m, h.normal, -d) * irr;
-                            icHit = true;
-                            nee = true;
-                        }
-                    } else if (createIC && rng.next() < fc.pc.irradianceCreateProb) {
-                        if (ncand < (uint32_t)kMaxNewCacheEntries) {
-                            float4 *c = pb.cand + 2 * ((size_t)pid * kMaxNewCacheEntries + ncand);
-                            c[0] = f4(h.worldPos, 0.0f);
-                            c[1] = f4(h.normal, 0.0f);
-                            ncand++;
-                        }
-                    }
-                }
-                if (!dead && splitOnFirst && depth == 1 && task.y < kMaxSplits) { // raytrace.rgen:1142-1146
-                    pushSplit(pb, pid, task, h, -d, thr * 0.5f, depth);
-                    thr = thr * 0.5f;
-                    taskDirty = true;
-                    hash = sigFold(hash, kSigSplit ^ 1u);
-                }
-                if (record && !icHit && !dead && grec.y != -1) { // raytrace.rgen:1153-1160
-                    recordSlots(pb, pid)[grec.y].distance += hit.x * __int_as_float(grec.z);
-                    if (!isMatAlmostDiscrete(m)) grec.y = -1;
-                }
-                if (dead) {
-                    isDone = true;
-                    nee = false;
-                }
-                doNee = nee && neeCapable(m.type) && S.lightCount > 0;
-                if (record) grec.w = grec.x; // the NEE light reaches the records made so far
+                // raytrace.rgen:1080-1139
+                wantIC = (useIC || (useADRRS && depth > 1)) && isICCapable(m.type, icOnGlossy);
             }
         }
         } // not a split vertex
+    }
+    // the wave's cache lookups, shared by its lanes
+    V3 irr = v3(0.0f);
+    bool icFound = false;
+    if (useIC || useADRRS) {
+        __shared__ IcWave icw[kShadeBlock / 64];
+        icFound = icQueryWave(IC, icp, icw[threadIdx.x >> 6], wantIC, h.worldPos, h.normal, irr);
+    }
+    if (vertex) {
+        if (wantIC) {
+            if (icFound) {
+                if (useADRRS) { // weight window against the cache's irradiance (1087-1116)
+                    const uint32_t pixel = (uint32_t)((b.firstPath + (pid - b.pathBase)) % b.npix);
+                    int nw;
+                    float q = weightWindow(rng, v3(pb.estimate[pixel]), irr, thr, adrrsS, nw);
+                    if (nw == 1) {
+                        if (rng.next() > q) { // the path dies here, before its NEE
+                            hash = sigFold(hash, kSigRRKill);
+                            dead = true;
+                        } else {
+                            thr = thr / q;
+                        }
+                    } else if (adrrsSplit) {
+                        const int room = kMaxSplits - task.y;
+                        if (nw - 1 > room) {
+                            nw = room + 1;
+                            q = (float)nw;
+                        }
+                        thr = thr / q;
+                        for (int k = 0; k < nw - 1; ++k) pushSplit(pb, pid, task, h, -d, thr, depth);
+                        taskDirty = true;
+                        hash = sigFold(hash, kSigSplit ^ (uint32_t)(nw - 1));
+                    }
+                } else {
+                    // a cache record ends the path after its NEE (1114-1122)
+                    hash = sigFold(hash, kSigCacheHit);
+                    res = res + thr * approxDiffuse(m, h.normal, -d) * irr;
+                    icHit = true;
+                    nee = true;
+                }
+            } else if (createIC && rng.next() < fc.pc.irradianceCreateProb) {
+                if (ncand < (uint32_t)kMaxNewCacheEntries) {
+                    float4 *c = pb.cand + 2 * ((size_t)pid * kMaxNewCacheEntries + ncand);
+                    c[0] = f4(h.worldPos, 0.0f);
+                    c[1] = f4(h.normal, 0.0f);
+                    ncand++;
+                }
+            }
+        }
+        if (!dead && splitOnFirst && depth == 1 && task.y < kMaxSplits) { // raytrace.rgen:1142-1146
+            pushSplit(pb, pid, task, h, -d, thr * 0.5f, depth);
+            thr = thr * 0.5f;
+            taskDirty = true;
+            hash = sigFold(hash, kSigSplit ^ 1u);
+        }
+        if (record && !icHit && !dead && grec.y != -1) { // raytrace.rgen:1153-1160
+            recordSlots(pb, pid)[grec.y].distance += hitT * __int_as_float(grec.z);
+            if (!isMatAlmostDiscrete(m)) grec.y = -1;
+        }
+        if (dead) {
+            isDone = true;
+            nee = false;
+        }
+        doNee = nee && neeCapable(m.type) && S.lightCount > 0;
+        if (record) grec.w = grec.x; // the NEE light reaches the records made so far
     }
     // ---- next event estimation, raytrace.rgen:601-731 (numNEE samples, multipleNEE 871-877)
     // A probe ray (the BSDF-sampled half of MIS) adds only if the first thing

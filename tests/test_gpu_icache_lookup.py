@@ -1,0 +1,67 @@
+"""Lookups that a wave shares among its lanes, against the oracle, at the
+sizes where the sharing has edges: no record, one record, records over more
+levels than are read at once (8), buckets with more pairs than one step tests
+(256) and lists longer than a wave, and frames whose waves are full, ragged or
+a single path.  Bars as in test_gpu_icache: paths that do not diverge from the
+FP64 oracle are within 1e-4 of it, and no more diverge than of the reference
+logic in FP32 (where a frame has enough paths for the share to mean
+something)."""
+import numpy as np
+import pytest
+
+import rtxamd
+import scenes
+from oracle.binding import OracleScene
+from parity import check_paths
+from rtxamd import abi
+from test_gpu_icache import cornell_state
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def cornell():
+    hs = rtxamd.HostScene.generate(abi.SCENE_CORNELL)
+    orc = OracleScene(abi, hs.desc())
+    return hs, orc, cornell_state(orc, hs)
+
+
+def variant(st, kind):
+    st = st.copy()
+    n = st.count
+    if kind == "none":
+        st.hdr.nextCacheSlot = 0
+    elif kind == "one":
+        st.hdr.nextCacheSlot = 1
+        st.spheres["radius"][0] *= 50.0
+        st.entries["harmonicR"][0] *= 50.0
+    elif kind == "levels":  # radii over twelve octaves
+        f = np.exp2((np.arange(n) % 12) - 8.0).astype(np.float32)
+        st.spheres["radius"][:n] *= f
+        st.entries["harmonicR"][:n] *= f
+    elif kind == "dense":  # every lookup meets hundreds of records
+        st.spheres["radius"][:n] *= 6.0
+        st.entries["harmonicR"][:n] *= 6.0
+    return st
+
+
+@pytest.mark.parametrize("kind", ["none", "one", "levels", "dense"])
+@pytest.mark.parametrize("w,h", [(1, 1), (13, 5), (64, 64)])
+def test_shared_lookups_match_oracle(renderer, cornell, kind, w, h):
+    hs, orc, st0 = cornell
+    st = variant(st0, kind)
+    renderer.ic_create(st.max_entries)
+    renderer.ic_write(st)
+    fp = scenes.params(hs, w, h, 1, maxDepth=8, enableMIS=1, useIrradianceCache=1, irradianceCreateProb=0.0,
+                       irradianceUpdateProb=0.0, irradianceCacheMinRadius=1e-3, sample_offset=3,
+                       flags=abi.RTX_FRAME_KEEP_PATHS | abi.RTX_FRAME_RESET_ACCUM)
+    ds = renderer.upload(hs)
+    try:
+        renderer.render(ds, fp)
+        rgb, sig = renderer.read_paths(w * h)
+    finally:
+        ds.close()
+    orgb, osig, _, _, _ = orc.ic_frame(fp, st.copy(), prec=64)
+    f32 = orc.ic_frame(fp, st.copy(), prec=32)[:2] if w * h >= 1000 else None
+    bar = 0.95 if w * h >= 1000 else 0.9
+    check_paths(f"shared lookups, {kind} {w}x{h}", rgb, sig, orgb, osig, f32, abs_same=bar, abs_within=bar)
