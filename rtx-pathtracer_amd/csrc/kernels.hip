@@ -745,8 +745,8 @@ RTX_DI void queueNee(const Queue &qs, const Queue &qp, V3 pos, const NeeRays &r,
 }
 
 // Register budget: two waves per SIMD (at most 256 VGPRs), three for a cache
-// frame's two classes (at most 168; 44 cache frames' kShade2: 139 ms with two,
-// 134 with three, 142 with four, which spills 170 registers).  The plain build
+// frame's two classes (at most 168; 44 cache frames' kShade2: 126 ms with two,
+// 118 with three, 124 with four).  The plain build
 // at 1080p: 0.61 ms a 4.1 M-path launch with two, 0.63 and 0.64 with three and
 // four.
 //
