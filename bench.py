@@ -18,7 +18,7 @@ Prints one JSON line.  `roofline` prices the dominant kernel (kTraceP, the
 persistent traversal that traces one bounce's extend rays together with the
 previous bounce's probe and shadow rays) by algorithmic bytes per ray = 32
 (ray) + 16 (hit) + nodes x node record + triangles x triangle record (the
-library's figures: 112 B read of a 128 B four-wide node, 48 B), with node and
+library's figures: an 80 B eight-wide node, 48 B), with node and
 triangle fetch counts from a counting pass of the identical (deterministic)
 workload and kernel times from HIP events on the library's stream.  `cpu_baseline` times the FP64 CPU
 restatement of the plain method on a pixel subsample of one sample plane.
