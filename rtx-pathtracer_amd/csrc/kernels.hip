@@ -1229,8 +1229,9 @@ __global__ __launch_bounds__(kShadeBlock, 2) void kShade(DevScene S, DevIC IC, D
 // Two classes of paths in one wavefront: ids below `split` are the class of
 // (fc, b), the others of (fc2, b2) (a frame's camera paths and the cache's
 // update sub-paths).  A wave takes one pass per class among its lanes.
+// The build with every feature takes two waves per SIMD, as kShade does.
 template <uint32_t F>
-__global__ __launch_bounds__(kShadeBlock, 3) void kShade2(DevScene S, DevIC IC, DevGuiding G,
+__global__ __launch_bounds__(kShadeBlock, F == kShadeAll ? 2 : 3) void kShade2(DevScene S, DevIC IC, DevGuiding G,
                                                        const FrameConst *__restrict__ fcp, BatchDesc b,
                                                        const FrameConst *__restrict__ fcp2, BatchDesc b2,
                                                        uint32_t split, PathBuffers pb, Queue qin, Queue qout,
@@ -1544,19 +1545,23 @@ void launchProbeResolve(hipStream_t s, const DevScene &S, const FrameConst *fc, 
 void launchShade(hipStream_t s, const DevScene &S, const DevIC &ic, const DevGuiding &g, const FrameConst *fc,
                  BatchDesc b, PathBuffers pb, Queue qin, Queue qout, Queue qs, Queue qp, int32_t *done, Counters *cnt,
                  int qsel, int blocks, uint32_t features, const PathClass2 *second) {
+    // The first build that holds every feature the frame uses: the ones frames
+    // mostly use have a build of their own, any other combination takes the full one.
+    const auto holds = [features](uint32_t f) { return (features & ~f) == 0u; };
     const dim3 grid(blocks), t(kShadeBlock);
     if (second) {
-        // a frame with its cache upkeep: no records, segments or learned cache
-        auto k = features & kShadeGuide ? kShade2<kShadeIC | kShadeGuide> : kShade2<kShadeIC>;
+        auto k = kShade2<kShadeAll>;
+        if (holds(kShadeIC)) k = kShade2<kShadeIC>;
+        else if (holds(kShadeIC | kShadeGuide)) k = kShade2<kShadeIC | kShadeGuide>;
         hipLaunchKernelGGL(k, grid, t, 0, s, S, ic, g, fc, b, second->fc, second->b, second->split, pb, qin, qout, qs,
                            qp, done, cnt, qsel);
         return;
     }
     auto k = kShade<kShadeAll>;
-    if (features == 0u) k = kShade<0u>;
-    else if ((features & ~kShadeIC) == 0u) k = kShade<kShadeIC>;
-    else if ((features & ~kShadeGuide) == 0u) k = kShade<kShadeGuide>;
-    else if ((features & ~kShadeNrc) == 0u) k = kShade<kShadeNrc>;
+    if (holds(0u)) k = kShade<0u>;
+    else if (holds(kShadeIC)) k = kShade<kShadeIC>;
+    else if (holds(kShadeGuide)) k = kShade<kShadeGuide>;
+    else if (holds(kShadeNrc)) k = kShade<kShadeNrc>;
     hipLaunchKernelGGL(k, grid, t, 0, s, S, ic, g, fc, b, pb, qin, qout, qs, qp, done, cnt, qsel);
 }
 void launchFinish(hipStream_t s, const FrameConst *fc, BatchDesc b, PathBuffers pb, const int32_t *done,
