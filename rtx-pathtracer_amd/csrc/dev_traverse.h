@@ -30,11 +30,7 @@ RTX_DI TravRay makeTravRay(V3 o, V3 d) {
     TravRay r;
     r.o = o;
     r.d = d;
-    // zero direction components get a tiny stand-in so slab tests never see 0*inf
-    float dx = d.x != 0.0f ? d.x : copysignf(1e-30f, d.x);
-    float dy = d.y != 0.0f ? d.y : copysignf(1e-30f, d.y);
-    float dz = d.z != 0.0f ? d.z : copysignf(1e-30f, d.z);
-    r.inv = v3(1.0f / dx, 1.0f / dy, 1.0f / dz);
+    r.inv = v3(1.0f / slabDirection(d.x), 1.0f / slabDirection(d.y), 1.0f / slabDirection(d.z));
     r.oinv = v3(o.x * r.inv.x, o.y * r.inv.y, o.z * r.inv.z);
     r.near1 = r.inv.x < 0.0f ? 0xAAu : 0x55u;
     r.near2 = r.inv.y < 0.0f ? 0xCCu : 0x33u;
@@ -215,8 +211,8 @@ RTX_DI int nearSlot(const TravRay &r, uint32_t set) {
 // the origin; rays from further away are covered by the factor 1 + 2 gamma_3
 // on the exit distance (Ize, "Robust BVH ray traversal", JCGT 2013).  So a box
 // the exact ray touches is never culled, and the hits do not depend on the
-// tree.  A NaN plane (0 * inf, inf - inf) constrains nothing: min and max
-// return their other operand.
+// tree.  A NaN plane (an overflow, planeOrigin; 0 * inf) constrains nothing:
+// min and max return their other operand.
 template <class SceneT, class Stack>
 RTX_DI void nodeStep(const SceneT &S, const TravRay &r, float tmin, float tmax, TravPos &pos, Stack &st) {
     const int slot = nearSlot(r, pos.group.y & 0xFFu);
@@ -230,9 +226,9 @@ RTX_DI void nodeStep(const SceneT &S, const TravRay &r, float tmin, float tmax, 
     const float sx = __uint_as_float((n0.w & 0xFFu) << 23) * r.inv.x;
     const float sy = __uint_as_float(((n0.w >> 8) & 0xFFu) << 23) * r.inv.y;
     const float sz = __uint_as_float(((n0.w >> 16) & 0xFFu) << 23) * r.inv.z;
-    const float ox = fmaf(__uint_as_float(n0.x), r.inv.x, -r.oinv.x);
-    const float oy = fmaf(__uint_as_float(n0.y), r.inv.y, -r.oinv.y);
-    const float oz = fmaf(__uint_as_float(n0.z), r.inv.z, -r.oinv.z);
+    const float ox = planeOrigin(__uint_as_float(n0.x), r.inv.x, r.oinv.x);
+    const float oy = planeOrigin(__uint_as_float(n0.y), r.inv.y, r.oinv.y);
+    const float oz = planeOrigin(__uint_as_float(n0.z), r.inv.z, r.oinv.z);
     const bool negx = r.near1 == 0xAAu, negy = r.near2 == 0xCCu, negz = r.near4 == 0xF0u;
     uint32_t miss = 0; // bit 7 - slot
 #pragma unroll
@@ -250,8 +246,7 @@ RTX_DI void nodeStep(const SceneT &S, const TravRay &r, float tmin, float tmax, 
                                          fmaf(ubyte(fz, k), sz, oz)),
                                    tmax);
             // the sign of exit - entry, shifted into the slots' misses
-            const float in = fmaf(tf, 1.0000004f, -tn);
-            miss = __builtin_amdgcn_alignbit(miss, __float_as_uint(in), 31);
+            miss = __builtin_amdgcn_alignbit(miss, __float_as_uint(entryMargin(tn, tf)), 31);
         }
     }
     const uint32_t imask = n0.w >> 24;
