@@ -82,9 +82,17 @@ RTX_BOX float planeOrigin(float p, float inv, float oinv) {
     return __builtin_fmaf(x, 0.0f, x);
 }
 
+// Entry and exit are each off by less than a factor 1 + gamma_4, gamma_4 =
+// 4 u / (1 - 4 u) with u = 2^-24 (Ize, "Robust BVH ray traversal", JCGT 2013):
+// u from 1 / d, u from the last FMA of a plane at l, and less than 2 u from
+// o inv and the origin plane's FMA, whose errors add up to (2 |o| + |p|) u in
+// units of |inv|.  The padding that packWide adds, 16 u (|l| + S), holds those
+// for |o| up to 7.5 S (o on the plane's axis); from farther away what is left
+// of them is below 2 u |l - o|.  So 1 + 10 u, which is above (1 + gamma_4) /
+// (1 - gamma_4), never culls a box that the exact ray touches, from any origin.
+constexpr float kExitSlack = 1.0000006f;
 // The box is entered unless this is negative (a NaN, of two infinities, counts
 // as entered).
-constexpr float kExitSlack = 1.0000004f;
 RTX_BOX float entryMargin(float tnear, float tfar) { return __builtin_fmaf(tfar, kExitSlack, -tnear); }
 
 constexpr int kLeafMaxPrims = 16;

@@ -286,12 +286,9 @@ struct Collapser {
 };
 
 // Pad a coordinate bound outwards by (|x| + S) 2^-20, S the scene's largest
-// coordinate magnitude (at least 1).  This covers FP32 hits that the
-// watertight test accepts just outside an edge, and the slab test's rounding:
-// it computes each plane distance as fma(l, 1/d, -o/d), whose point along the
-// axis lies within (|l| + 2|o|) 2^-24 (1 + 2^-23) of the plane, below
-// 16 (|l| + S) 2^-24 for every ray that starts within 7.5 S of the origin
-// (every secondary ray, and cameras up to 7 scene sizes away).
+// coordinate magnitude (at least 1): the FP32 hits that the watertight test
+// accepts just outside an edge.  packWide pads as much again for the box
+// test's rounding (kExitSlack, bvh.h).
 inline float padLo(float x, float S) { return x - (std::fabs(x) + S) * 9.5367431640625e-07f; }
 inline float padHi(float x, float S) { return x + (std::fabs(x) + S) * 9.5367431640625e-07f; }
 

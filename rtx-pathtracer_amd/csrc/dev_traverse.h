@@ -205,14 +205,11 @@ RTX_DI int nearSlot(const TravRay &r, uint32_t set) {
 // [tmin, tmax], and the entered ones become the group and the leaves to test.
 // With no inner child entered the next stack entry becomes the group.
 //
-// A box plane is one FMA, fma(q, 2^e inv, p inv - o inv).  Its error is below
-// (4 |o| + |p| + 2 |l|) 2^-24 in units of |inv| for a plane at l, which the
-// boxes' padding of (|x| + S) 2^-19 covers for rays that start within 7 S of
-// the origin; rays from further away are covered by the factor 1 + 2 gamma_3
-// on the exit distance (Ize, "Robust BVH ray traversal", JCGT 2013).  So a box
-// the exact ray touches is never culled, and the hits do not depend on the
-// tree.  A NaN plane (an overflow, planeOrigin; 0 * inf) constrains nothing:
-// min and max return their other operand.
+// A box plane is one FMA, fma(q, 2^e inv, planeOrigin).  Its rounding is covered
+// by the boxes' padding and by the slack on the exit distance (kExitSlack,
+// bvh.h), so a box the exact ray touches is never culled, and the hits do not
+// depend on the tree.  A NaN plane (an overflow, planeOrigin; 0 * inf) constrains
+// nothing: min and max return their other operand.
 template <class SceneT, class Stack>
 RTX_DI void nodeStep(const SceneT &S, const TravRay &r, float tmin, float tmax, TravPos &pos, Stack &st) {
     const int slot = nearSlot(r, pos.group.y & 0xFFu);
