@@ -330,7 +330,6 @@ void buildBvh(const float *tv, uint32_t numTris, BvhBuildResult &out) {
     out.binaryDepth = b.maxDepth + 1;
     Collapser c{b.nodes, {}, 0};
     c.collapse(0, 1);
-    if (3u * c.maxDepth > (uint32_t)kStackCapacity) throw std::runtime_error("BVH too deep for the traversal stack");
     out.nodes = std::move(c.out);
     out.primOrder = std::move(b.order);
     out.maxDepth = c.maxDepth;

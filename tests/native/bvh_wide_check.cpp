@@ -17,8 +17,10 @@ static void check(const std::vector<float> &v, const char *name) {
     const uint32_t n = (uint32_t)(v.size() / 9);
     BvhBuildResult r;
     WideBvh w;
-    try { buildBvh(v.data(), n, r); } catch (std::exception &e) { printf("%s: build threw %s\n", name, e.what()); return; }
-    packWide(r, w);
+    try {
+        buildBvh(v.data(), n, r);
+        packWide(r, w);
+    } catch (std::exception &e) { printf("%s: threw %s\n", name, e.what()); ++fails; return; }
     std::vector<int> cover(n, 0);
     std::vector<bool> reached(w.nodes.size(), false);
     if (w.triOrder.size() != n || w.maxDepth > (uint32_t)kStackCapacity) { printf("%s: %zu triangles, depth %u\n", name, w.triOrder.size(), w.maxDepth); ++fails; return; }
@@ -85,6 +87,7 @@ int main() {
     { auto v = rnd(3000, 1); for (size_t i = 0; i < v.size(); i += 3) v[i] *= 1e30f; check(v, "huge"); }
     { auto v = rnd(3000, 1); for (size_t i = 0; i < v.size(); i += 3) v[i] *= 1e-38f; check(v, "flat"); }
     { std::vector<float> w; for (int i = 0; i < 60000; ++i) { float x = std::ldexp(1.0f, -(i % 120)); float t[9] = {x, x, x, x * 2, x, x, x, x * 2, x}; w.insert(w.end(), t, t + 9); } check(w, "geometric60000"); }
+    { std::vector<float> w; for (int i = 0; i < 60000; ++i) { const float x = std::pow(4.0f, -(float)(i % 60)) * ((i / 60) % 2 ? -1.0f : 1.0f); float t[9] = {x, x, x, x * 2, x, x, x, x * 2, x}; w.insert(w.end(), t, t + 9); } check(w, "nested60000"); } // a four-wide tree of more than 21 levels
     printf("fails %d\n", fails);
     return fails != 0;
 }
