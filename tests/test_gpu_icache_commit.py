@@ -41,6 +41,11 @@ def test_commit_matches_job_order(renderer, entries, frames, size, create, updat
     assert len(jobs) > 0 and got.count == c
     assert np.array_equal(ref.entries["numUpdates"][:c], got.entries["numUpdates"][:c])
     assert np.allclose(got.spheres["center"][:c], ref.spheres["center"][:c], rtol=0, atol=1e-6)
+    assert np.allclose(got.entries["normal"][:c], ref.entries["normal"][:c], rtol=0, atol=1e-6)
+    # a mean of at most 200 positive terms, in both the same order: rounding below 200 x 2^-24 = 1.2e-5
+    for a, b in ((got.entries["harmonicR"], ref.entries["harmonicR"]), (got.spheres["radius"], ref.spheres["radius"])):
+        assert (b[:c] > 0).all() and np.allclose(a[:c], b[:c], rtol=1.2e-5, atol=0)
+    assert (got.hdr.nextCacheSlot, got.hdr.maxCaches) == (ref.hdr.nextCacheSlot, ref.hdr.maxCaches)
     for f in ("color", "rotGrad", "transGrad"):
         a, b = got.entries[f][:c].astype(np.float64), ref.entries[f][:c].astype(np.float64)
         # 1e-4 of the record's scale.  A gradient is a sum of up to 400 signed

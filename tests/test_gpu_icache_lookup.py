@@ -5,7 +5,9 @@ levels than are read at once (8), buckets with more pairs than one step tests
 a single path.  Bars as in test_gpu_icache: paths that do not diverge from the
 FP64 oracle are within 1e-4 of it, and no more diverge than of the reference
 logic in FP32 (where a frame has enough paths for the share to mean
-something)."""
+something).  A wrong term in a few shared lookups would hide in those shares:
+so frames are also compared, bit for bit, with the same paths shaded in waves
+that hold one path alone."""
 import numpy as np
 import pytest
 
@@ -63,5 +65,34 @@ def test_shared_lookups_match_oracle(renderer, cornell, kind, w, h):
         ds.close()
     orgb, osig, _, _, _ = orc.ic_frame(fp, st.copy(), prec=64)
     f32 = orc.ic_frame(fp, st.copy(), prec=32)[:2] if w * h >= 1000 else None
-    bar = 0.95 if w * h >= 1000 else 0.9
-    check_paths(f"shared lookups, {kind} {w}x{h}", rgb, sig, orgb, osig, f32, abs_same=bar, abs_within=bar)
+    # the reference logic in FP32 diverges on 0.3 to 1.4% of the 4096 paths and is past 1e-4 on 0.1 to
+    # 0.25% of the others; of 65 paths one may do either
+    check_paths(f"shared lookups, {kind} {w}x{h}", rgb, sig, orgb, osig, f32, abs_same=0.98, abs_within=0.98)
+
+
+@pytest.mark.parametrize("kind", ["one", "levels", "dense"])
+@pytest.mark.parametrize("w,h,batches", [(13, 5, (1, 7, 64)), (64, 64, (63, 1000))])
+def test_sharing_changes_no_bit(renderer, cornell, kind, w, h, batches):
+    """A lookup adds its records' terms in the order of its own walk, whatever
+    its wave's other lanes look up: frames shaded in batches of one path (each
+    lookup alone in its wave), of a ragged wave or of several waves equal the
+    frame in one batch bit for bit."""
+    hs, _, st0 = cornell
+    st = variant(st0, kind)
+    renderer.ic_create(st.max_entries)
+    renderer.ic_write(st)
+    ds = renderer.upload(hs)
+    out = []
+    try:
+        for batch in (0,) + batches:
+            fp = scenes.params(hs, w, h, 2, maxDepth=8, enableMIS=1, useIrradianceCache=1, irradianceCreateProb=0.0,
+                               irradianceUpdateProb=0.0, irradianceCacheMinRadius=1e-3, useIrradianceGradients=1,
+                               sample_offset=5, flags=abi.RTX_FRAME_RESET_ACCUM)
+            fp.batchPaths = batch
+            renderer.render(ds, fp)
+            out.append(renderer.read_image(w, h).view(np.uint32))
+    finally:
+        ds.close()
+    assert out[0].view(np.float32)[..., :3].max() > 0
+    for o in out[1:]:
+        assert np.array_equal(o, out[0])
