@@ -1258,7 +1258,7 @@ int rtx_render(rtx_ctx *ctx, const rtx_scene *scene, const rtx_frame_params *p, 
             if (nrc) // the paths that ended into the learned cache: throughput x cache
                 timed(kClsShade, [&] {
                     launchNrcInfer(s, ctx->nrc, ctx->pb.nrcQuery, NrcRows{1, ctx->pb.nrcQueryStride}, b.numPaths,
-                                   ctx->pb.nrcQueryCount, ctx->nrcFeat, nullptr,
+                                   ctx->pb.nrcQueryCount, ctx->nrcFeat, kNrcInferRows, nullptr,
                                    ctx->pb.nrcQueryAux, ctx->pb.out, 2 * ctx->cuCount,
                                    NrcSelfTrain{ctx->pb.thr, ctx->pb.nrcPath,
                                                 fc.nrcSuffix ? ctx->pb.nrcTrainTarget : nullptr, kFlagNrcTrainEnd});
@@ -2267,14 +2267,14 @@ int rtx_nrc_infer(rtx_ctx *ctx, const rtx_nrc_input *in, size_t n, float *rgb) t
     CHECK_HIP(ctx, hipSetDevice(ctx->device));
     std::vector<void *> tmp;
     float4 *inD = nullptr, *outD = nullptr;
-    uint32_t *feat = nullptr;
     int rc = nrcUpload(ctx, in, nullptr, n, tmp, &inD, nullptr);
     if (rc == RTX_OK) {
-        hipError_t e = devAlloc(&outD, n, tmp);
-        if (e == hipSuccess) e = devAlloc(&feat, (size_t)kNrcMaxLevels * std::min(n, kNrcInferRows), tmp);
+        // the results, then a slice's features, in one allocation
+        const size_t featRows = std::min(n, kNrcCallRows);
+        hipError_t e = devAlloc(&outD, n + kNrcMaxLevels / 4 * featRows, tmp);
         if (e == hipSuccess) {
-            launchNrcInfer(ctx->stream, ctx->nrc, inD, NrcRows{4, 1}, (uint32_t)n, nullptr, feat, outD, nullptr,
-                           nullptr, 2 * ctx->cuCount);
+            launchNrcInfer(ctx->stream, ctx->nrc, inD, NrcRows{4, 1}, (uint32_t)n, nullptr,
+                           reinterpret_cast<uint32_t *>(outD + n), featRows, outD, nullptr, nullptr, 2 * ctx->cuCount);
             e = hipGetLastError();
         }
         std::vector<float4> out(n);

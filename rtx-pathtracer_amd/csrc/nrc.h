@@ -81,14 +81,16 @@ struct NrcSelfTrain {
     float4 *target;   // NULL: no self-training
     uint32_t endFlag;
 };
-// Inference encodes and evaluates at most this many rows at a time, which
-// bounds the features between the two kernels (256 MB).
-constexpr size_t kNrcInferRows = 1u << 22;
+// Inference encodes and evaluates a slice of rows at a time, which bounds the
+// features between the two kernels: a render's 2^22 rows (256 MB, kept with its
+// path buffers), and 2^18 (16 MB) in rtx_nrc_infer, which allocates them on each
+// call (a million rows: 4.76 ms; 4.98 with the features of all of them, 61 MB).
+constexpr size_t kNrcInferRows = 1u << 22, kNrcCallRows = 1u << 18;
 // n rows, or *count rows (at most n) when count is given; feat: work memory,
-// kNrcMaxLevels x min(n, kNrcInferRows) words
+// kNrcMaxLevels x featRows words
 void launchNrcInfer(hipStream_t s, const NrcBuffers &nb, const float4 *in, NrcRows rows, uint32_t n,
-                    const uint32_t *count, uint32_t *feat, float4 *out, const float4 *aux, float4 *pathOut, int blocks,
-                    NrcSelfTrain st = {});
+                    const uint32_t *count, uint32_t *feat, size_t featRows, float4 *out, const float4 *aux,
+                    float4 *pathOut, int blocks, NrcSelfTrain st = {});
 // Rows (queries, training vertices) are rtx_nrc_input records, 4 float4 each:
 // (pos, roughness), (dir, -), (normal, -), (albedo, -).
 // Forward with saved activations, the loss gradient, the backward pass, the

@@ -533,12 +533,12 @@ static void launchEncode(hipStream_t s, const NrcBuffers &nb, const float4 *in, 
 }
 
 void launchNrcInfer(hipStream_t s, const NrcBuffers &nb, const float4 *in, NrcRows rows, uint32_t n,
-                    const uint32_t *count, uint32_t *feat, float4 *out, const float4 *aux, float4 *pathOut, int blocks,
-                    NrcSelfTrain st) {
+                    const uint32_t *count, uint32_t *feat, size_t featRows, float4 *out, const float4 *aux,
+                    float4 *pathOut, int blocks, NrcSelfTrain st) {
     NrcBuffers v = nb; // inference reads the moving average's copies
     v.gridBf16 = nb.gridBf16Ema;
     v.wFwd = nb.wFwdEma;
-    const size_t stride = n < kNrcInferRows ? n : kNrcInferRows;
+    const size_t stride = n < featRows ? n : featRows;
     for (size_t r0 = 0; r0 < n; r0 += stride) {
         const NrcRange range{(uint32_t)(n - r0 < stride ? n - r0 : stride), count, (uint32_t)r0};
         const int tiles = (int)((range.n + kNrcRowsPerBlock - 1) / kNrcRowsPerBlock);

@@ -2,8 +2,8 @@
 levels, and the table gradient, whose lanes share a row: at 1, 8, 9 and 16
 levels (none, one or two levels an eighth), tables small enough that only the
 hash is used and large enough that dense levels are among them, and row counts
-around the 16-, 128- and 256-row pieces; and inference in slices (more than
-2^22 rows) against the same rows alone."""
+around the 16-, 128- and 256-row pieces; and inference in slices (of 2^18
+rows) against the same rows alone."""
 import numpy as np
 import pytest
 import torch
@@ -64,9 +64,9 @@ def test_encoding_and_table_gradient(renderer, levels, log2, rows):
     assert np.linalg.norm(ggrid - want) <= 2.0 ** -7 * np.linalg.norm(want)
 
 
-def test_inference_in_slices(renderer):
+@pytest.mark.parametrize("n", [1 << 18, (1 << 18) + 1, (1 << 22) + 77])
+def test_inference_in_slices(renderer, n):
     renderer.nrc_create(LO, HI, seed=3, levels=8, log2TableSize=12)
-    n = (1 << 22) + 77
     rng = np.random.default_rng(1)
     x = np.tile(random_inputs(4099, LO, HI, rng), ((n + 4098) // 4099, 1))[:n]
     got = renderer.nrc_infer(x)
