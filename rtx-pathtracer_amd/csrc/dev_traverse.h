@@ -196,10 +196,12 @@ RTX_DI int nearSlot(const TravRay &r, uint32_t set) {
 // The four-wide FP32 nodes before these took seven 16-byte loads and 28
 // visits a ray in the 262,144-triangle room, and the loads' address
 // processing bounded the launch (TA busy 95%, 0.70 cache accesses a cycle and
-// CU).  These take five loads and 19 visits (TA busy 76%); the launch is bound
-// by vector instructions, 48 conversions and 48 FMAs of a visit's 180 first
-// (v_perm pairs into v_fma_mix instead of conversions measured the same):
-// 1.49 -> 0.97 ms for 2 x 1080p paths (1.85 before the rays went out in chunks).
+// CU).  These take five loads and 19 visits (TA busy 81%, 0.81 accesses); the
+// launch is bound by vector instructions, 0.30 a SIMD and cycle with half the
+// lanes active, 48 conversions and 48 FMAs of a visit's 180 first (v_perm pairs
+// into v_fma_mix instead of conversions measured the same): 1.49 -> 0.97 ms for
+// 2 x 1080p paths (1.85 before the rays went out in chunks), 0.90 in the
+// present build.
 // One node visit: the next of the group's children in the ray's order is
 // taken (the rest pushed), its children's boxes are tested against
 // [tmin, tmax], and the entered ones become the group and the leaves to test.
